@@ -151,6 +151,8 @@ struct RasterBufs {
   float* T;
   uint32_t* end;
   float4* gC;             // dL/dC, w = valid
+  uint64_t* took;         // per 64-key chunk of a tile and wave: the keys that a lane of the wave took
+                          // (training: written by the forward, read by the backward)
   const uint32_t* tgt;    // packed RGBA8 targets (all views)
   double* stats;          // [0] sum |err|^2, [1] loss, [2] valid pixels
 };
@@ -167,6 +169,7 @@ __device__ __forceinline__ RasterBufs global_bufs(const RasterBufs& s) {
   r.T = gs_global(s.T);
   r.end = gs_global(s.end);
   r.gC = gs_global(s.gC);
+  r.took = gs_global(s.took);
   r.tgt = gs_global(s.tgt);
   r.stats = gs_global(s.stats);
   return r;
@@ -219,6 +222,9 @@ struct RasterShape {
   int tile, batch;
 };
 bool raster_shape_ok(int tile, int batch);
+// bytes of RasterBufs::took for views of up to w x h pixels and `keys` sorted
+// keys, enough at every raster shape
+size_t raster_took_bytes(int w, int h, int64_t keys);
 
 // loss: 0 none (view render), 1 Charbonnier fused into the forward pass,
 // 2 forward only, loss computed by a separate kernel

@@ -106,6 +106,34 @@ GS_HD float gs_expf_mid(float x) {
 // polynomial; at most 2 ulp from the correctly rounded e^x on every float of
 // [-87, 0] (gs_expf: at most 1), inside WGSL's 3 + 2|x| ulp for exp.
 GS_HD float gs_expf_raster(float xc) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  // The same operations on e = -xc in [0, 87], arranged for the VALU: on
+  // gfx950 an add, multiply or FMA of registers and literals issues at twice
+  // the rate of v_rndne_f32, v_cvt_i32_f32 or an instruction with a scalar
+  // operand.
+  // k = round(x/ln2) by adding and subtracting 1.5 * 2^23, which leaves k in
+  // the sum's low bits: the same integer as rintf's (both round ties to
+  // even); where it is zero its sign may differ, which no later operation
+  // sees (p = 1 at r = +-0).
+  const float e = -xc;
+  const float ks = e * -1.44269502162933349609375f + 12582912.0f;
+  const float kf = ks - 12582912.0f;
+  // n = -r, and the polynomial's steps with alternating signs, so that only
+  // literals carry a sign (rounding is symmetric: every value is the other
+  // form's or its exact negation)
+  float n = fmaf(kf, 0.693145751953125f, e);
+  n = fmaf(kf, 1.428606765330187045e-06f, n);
+  const float p1 = fmaf(gs_u2f(0x3c0840d6u), n, -gs_u2f(0x3d2b9b09u));
+  const float p2 = fmaf(p1, n, gs_u2f(0x3e2aabc8u));
+  const float p3 = fmaf(p2, n, -gs_u2f(0x3efffeeeu));
+  const float p4 = fmaf(p3, n, 1.0f);
+  const float p = fmaf(-p4, n, 1.0f);
+  // p 2^k by adding k to the exponent field (the shift drops the magic sum's
+  // own bits). Equal to the product below: k = -126 only for x < -86.99, where
+  // r >= 0.337 and p >= 1.4, and p >= 0.707 otherwise, so p 2^k is always
+  // normal and exact either way.
+  return gs_u2f((gs_f2u(ks) << 23) + gs_f2u(p));
+#else
   const float kf = rintf(xc * 1.44269502162933349609375f);
   float r = fmaf(kf, -0.693145751953125f, xc);
   r = fmaf(kf, -1.428606765330187045e-06f, r);
@@ -115,14 +143,7 @@ GS_HD float gs_expf_raster(float xc) {
   p = fmaf(p, r, gs_u2f(0x3efffeeeu));       // 4.9999183e-01
   p = fmaf(p, r, 1.0f);
   p = fmaf(p, r, 1.0f);
-  const int k = (int)kf;
-#if defined(__HIP_DEVICE_COMPILE__)
-  // p 2^k in one v_ldexp_f32 instead of building 2^k and multiplying. Both
-  // are exact and equal: k = -126 only for x < -86.99, where r >= 0.337 and
-  // p >= 1.4, and p >= 0.707 otherwise, so p 2^k is always normal.
-  return __builtin_amdgcn_ldexpf(p, k);
-#else
-  return p * gs_u2f((uint32_t)(k + 127) << 23);
+  return p * gs_u2f((uint32_t)((int)kf + 127) << 23);
 #endif
 }
 

@@ -27,10 +27,12 @@
 // its pixels down to the first key (each wave from the largest `end` of its
 // own pixels), recomputing each pixel's transmittance
 // in front of a splat from the stored final T (Tb = Ta/(1-a), through one
-// reciprocal that also scales the colour-behind sum S).
+// reciprocal that also scales the colour-behind sum S). A wave visits exactly
+// the keys that some lane of it took in the forward, which leaves one word per
+// 64 keys and wave for this (RasterBufs::took).
 // Per key, the 10 screen-space gradient terms of the wave's 64 pixels are
-// summed with a transpose reduction of lane exchanges (below) and added to
-// the Gaussian's accumulator with one atomic per term per wave:
+// summed (DPP adds, then the wave's own LDS scratch; WaveRed below) and added
+// to the Gaussian's accumulator with one atomic per term per wave:
 //   GS_ACCUM_FIXED: each pixel's term is converted to i32 first,
 //                   i32(clamp(v * 16384, -1e9, 1e9)), exactly as the
 //                   reference's atomicAdd on atomic<i32> (shaders.js:529-541);
@@ -47,6 +49,16 @@
 // one LDS array, and the backward stages the tile's records again while
 // they are still in L2 from the forward. Renders, and the L1 + D-SSIM loss
 // (whose gradient needs neighbouring pixels), run the passes apart.
+//
+// What bounds both visit loops is instruction issue: vector instructions
+// where the chip is full, and on small images, with about one wave per SIMD,
+// every instruction, scalar ones included (~4 cycles each there). So the
+// masks of a visit live in scalar registers, with one instruction to clear a
+// bit, and the records of a chunk lie in the order of the walk, which makes
+// it a find-first-bit both ways. Measured with the reduction through LDS and
+// the took words (1M Gaussians, 1600x900, ~3.25M keys): forward and backward
+// in one launch 626 -> 538 us; 8 views at once 4.32 -> 3.84 ms; the forward
+// alone at 1237x933, 2.0M keys, 155 -> 132 us, the backward 439 -> 382.
 #include <type_traits>
 
 #include "gs_kernels.h"
@@ -89,14 +101,15 @@ struct Shape {
 
 // LDS of the raster passes, carved from one array that the kernel declares,
 // so a launch that runs both passes holds the larger layout, not both.
-// Forward: records sA, sB, sC (16 B each per key), the chunk masks, the loss
-// partials; backward: records sA-sD, the chunk masks, the block's largest
-// end. Sizes in float4.
+// Forward: records sA, sB, sC (16 B each per key), the chunk masks per
+// quadrant, the loss partials; backward: records sA-sD, the chunk masks per
+// wave, the block's largest end. Sizes in float4.
+constexpr int kRedStride = 68;   // words between a wave's 64-word rows (see WaveRed)
 template <class S>
 struct RasterLds {
-  static constexpr int kMaskBytes = S::kChunks * S::kMasks * 8;
-  static constexpr int kFwd = 3 * S::B + (kMaskBytes + 3 * S::kWaves * 8 + 15) / 16;
-  static constexpr int kBwd = 4 * S::B + (kMaskBytes + 4 + 15) / 16;
+  static constexpr int kFwd = 3 * S::B + (S::kChunks * S::kMasks * 8 + 3 * S::kWaves * 8 + 15) / 16;
+  static constexpr int kRed = S::kWaves * 5 * kRedStride / 4;   // the waves' reduction scratch
+  static constexpr int kBwd = 3 * S::B + kRed + (S::kChunks * S::kWaves * 8 + 4 + 15) / 16;
   static constexpr int kBoth = kFwd > kBwd ? kFwd : kBwd;
 };
 
@@ -141,6 +154,17 @@ __device__ __forceinline__ void store_masks(uint32_t cover, uint64_t* m) {
   }
 }
 
+// m without bit `bit`, in one scalar instruction (the compiler takes two or three)
+__device__ __forceinline__ void clear_bit(uint64_t& m, int bit) {
+  asm("s_bitset0_b64 %0, %1" : "+s"(m) : "s"(bit));
+}
+
+// the same when `mask` is empty (left to the compiler: five instructions)
+__device__ __forceinline__ void clear_bit_if_none(uint64_t& m, int bit, uint64_t mask) {
+  asm("s_cmp_lg_u64 %1, 0\n\ts_cbranch_scc1 .Lgs_some%=\n\ts_bitset0_b64 %0, %2\n.Lgs_some%=:"
+      : "+s"(m) : "s"(mask), "s"(bit) : "scc");
+}
+
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
@@ -168,6 +192,10 @@ __device__ __forceinline__ const T& lds_at(const void* base, uint32_t off) {
 // e is finite (bounded conic and offsets), where med3 equals the pair.
 __device__ __forceinline__ float clamp_e(float e) { return __builtin_amdgcn_fmed3f(e, 0.0f, 87.0f); }
 
+__device__ __forceinline__ float max3abs(float a, float b, float c) {
+  return fmaxf(fmaxf(fabsf(a), fabsf(b)), fabsf(c));
+}
+
 // 1/x for x in [2^-9, 1]: hardware reciprocal estimate plus one Newton step
 // with fused residual. Equal to IEEE 1.0f/x for all 75,497,473 floats of that
 // range (exhaustive check on gfx950); callers guarantee the range.
@@ -187,10 +215,21 @@ __device__ __forceinline__ float4 record_colour(int recFmt, const float4& r1, fl
   return make_float4(dec16<1>(rg), dec16<1>(rg >> 16), dec16<1>(bl), w);
 }
 
+// First word (of one per wave) of RasterBufs::took for 64-key chunk `c`
+// (below the tile's keys / 64, rounded up) of the tile whose keys start at s.
+// Tiles lie in key order, so the rows of two
+// tiles never overlap: s / 64 grows by at least the earlier tile's chunks
+// less one, and the tile index by one.
+template <class S>
+__device__ __forceinline__ size_t took_word(uint32_t s, int tile, uint32_t c) {
+  return ((size_t)(s >> 6) + (uint32_t)tile + c) * S::kWaves;
+}
+
 // One tile of the forward pass, by the whole 256-thread block. The block's
 // threads must all call it (it synchronises), and nothing else may use the
-// block's LDS until every thread has returned.
-template <class S, int kLoss>
+// block's LDS until every thread has returned. kTook: record the keys each
+// wave's lanes take, for the backward.
+template <class S, int kLoss, bool kTook>
 __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, const RasterBufs& b, int tile,
                                                 float4* lds, PixelState* out = nullptr) {
   float4* const sA = lds;              // mx, my, A, B
@@ -209,9 +248,11 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
   if (out) *out = PixelState{make_float4(0.0f, 0.0f, 0.0f, 0.0f), 0.0f, s};
   float T = 1.0f, C0 = 0.0f, C1 = 0.0f, C2 = 0.0f;
   uint32_t end = s;
-  bool done = !inside;
+  // lanes still compositing, in scalar registers: a lane is done once outside
+  // the image or once T < 1e-4
+  uint64_t run = wave_ballot(inside);
   for (uint32_t base = s; base < e; base += S::B) {
-    if (__syncthreads_count(!done) == 0) break;
+    if (__syncthreads_or(run != 0ull) == 0) break;
     // wave w stages chunks w, w + kWaves, ... (lane l: key 64 c + l)
     for (int c = wv; c < S::kChunks; c += S::kWaves) {
       const int j = 64 * c + lane;
@@ -238,33 +279,33 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
     }
     __syncthreads();
     const uint32_t cnt = min((uint32_t)S::B, e - base);
-    // lanes still compositing; a lane is done once outside the image or
-    // once T < 1e-4, so the vote is kept current with one compare per splat
-    uint64_t run = wave_ballot(!done);
     if (run != 0ull) {
-      uint32_t term = 0xffffffffu;  // batch index of this pixel's last splat
       for (int c = 0; c < S::kChunks; c++) {
         uint64_t m = uniform64(sMask[c][mslot]);
+        uint64_t took = m;   // kTook: keys of the chunk that some lane takes
         while (m) {
-          const int j = c * 64 + (int)__builtin_ctzll(m);
-          m &= m - 1ull;
-          // Straight-line for all lanes; only lanes that take the splat
-          // (not done, inside the cutoff, alpha >= A_MIN) update their state.
-          const uint32_t jo = lds_offset((uint32_t)j * 16u);
-          const float4 a = lds_at<float4>(sA, jo);
-          const float2 bb = lds_at<float2>(sB, jo);   // C, opa*comp
-          asm volatile("" ::"v"(bb.y));                // one 8-byte read
+          const int bit = (int)__builtin_ctzll(m);
+          clear_bit(m, bit);
+          // Only lanes that take the splat (still running, inside the cutoff,
+          // alpha >= A_MIN) update their state; the wave leaves as soon as
+          // there is none. The masks are combined in scalar registers.
+          const uint32_t jo = lds_offset((uint32_t)bit * 16u);
+          const float4 a = lds_at<float4>(sA + 64 * c, jo);
+          const float2 bb = lds_at<float2>(sB + 64 * c, jo);   // C, opa*comp
+          asm volatile("" ::"v"(bb.y));                         // one 8-byte read
           const float dx = px - a.x, dy = py - a.y;
           const float t2 = fmaf(bb.x * dy, dy, (a.z * dx) * dx);
           // clamped to [0, 87]: an exponent above 87 > eCut is never taken,
           // and the exp below needs its argument in [-87, 0]
           const float ee = clamp_e(fmaf(0.5f, t2, (a.w * dx) * dy));
-          const bool live = !done && ee <= cut.eCut;
-          if ((run & wave_ballot(ee <= cut.eCut)) != 0ull) {
+          const uint64_t live = run & wave_ballot(ee <= cut.eCut);
+          uint64_t take = 0ull;
+          if (live != 0ull) {
             const float araw = bb.y * gs_expf_raster(-ee);
             const float alpha = fminf(0.99f, araw);
-            if (live && alpha >= cut.aMin) {
-              const float4 c4 = lds_at<float4>(sC, jo);
+            take = live & wave_ballot(alpha >= cut.aMin);
+            if (__builtin_amdgcn_inverse_ballot_w64(take)) {
+              const float4 c4 = lds_at<float4>(sC + 64 * c, jo);
               const float w = T * alpha;
               C0 = fmaf(w, c4.x, C0);
               C1 = fmaf(w, c4.y, C1);
@@ -274,18 +315,20 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
             // T only falls here, so a lane reaches T < 1e-4 on this splat
             // exactly when it is still running and now below; that happens
             // once per pixel, so its bookkeeping sits behind a scalar branch
-            const bool fin = T < 1e-4f;
-            const uint64_t left = run & ~wave_ballot(fin);
-            if (left != run) {
-              if (fin && !done) { done = true; term = (uint32_t)j; }
-              run = left;
-              if (run == 0ull) { m = 0ull; c = S::kChunks; }
+            const uint64_t fin = run & wave_ballot(T < 1e-4f);
+            if (fin != 0ull) {
+              if (__builtin_amdgcn_inverse_ballot_w64(fin)) end = base + (uint32_t)(64 * c + bit) + 1u;
+              run &= ~fin;
+              if (run == 0ull) m = 0ull;
             }
           }
+          if (kTook) clear_bit_if_none(took, bit, take);
         }
+        if (kTook && lane == 0 && 64u * (uint32_t)c < cnt)
+          b.took[took_word<S>(s, tile, ((base - s) >> 6) + (uint32_t)c) + wv] = took;
+        if (run == 0ull) break;
       }
-      if (term != 0xffffffffu) end = base + term + 1u;
-      else if (!done) end = base + cnt;
+      if (__builtin_amdgcn_inverse_ballot_w64(run)) end = base + cnt;
     }
   }
   double st0 = 0.0, st1 = 0.0, st2 = 0.0;
@@ -338,28 +381,34 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
   }
 }
 
-// ---- wave transpose reduction of a visit's 10 values (VALU lane exchanges) ----
-// Six halving steps, one per lane-index bit, in this order: l ^ 15 (row_mirror,
-// across bit 3), l ^ 7 (row_half_mirror, bit 2), l ^ 2 and l ^ 1 (quad_perm),
-// l ^ 16 (v_permlane16_swap), l ^ 32 (v_permlane32_swap). In each a lane
-// keeps one half of its values and adds its partner's copy of that half (an
-// odd count is padded with a zero), so after the last step each slot's
-// 64-lane total sits in exactly one lane and every other lane holds a
-// padding zero. The slot each lane ends with is measured once per kernel by
-// running the network on constants.
-//
-// The first two steps separate the lower and upper half by 4-lane bank
-// (lanes 0-7 / 8-15 of a row, then 0-3, 8-11 / 4-7, 12-15), so they run as
-// two DPP adds per output, each writing one half through the DPP bank mask:
-// no selects. They run on each visit's terms as they are made (10 -> 5 -> 3
-// values per lane); the last four steps run once per two visits on their
-// 3 + 3 values (keep/send selects and one DPP add per output for the quad
-// steps; the cross-row swaps on one value each). The asm blocks start with
-// two wait states for the DPP read of a value the previous VALU instruction
-// wrote, and end with two for a DPP read of their results that follows.
-// Every step runs with all 64 lanes active (the visit loop branches only on
-// wave-uniform votes, and every wave of a block is full): a DPP add whose
-// source lane were inactive would leave its output unwritten.
+// ---- wave reduction of a visit's 10 values ----
+// A visit's terms are summed over the wave's 64 lanes in two steps:
+//  1. l ^ 15 (row_mirror, across bit 3 of the lane index) as two DPP adds per
+//     output, each writing one half of the row through the DPP bank mask (no
+//     selects): lanes 0-7 of each 16-lane row keep values 0-4, lanes 8-15
+//     values 5-9, so 10 values become 5 per lane;
+//  2. through the wave's own LDS scratch: register i goes to word 68 i +
+//     lane, so the 8 words of one value and row lie next to each other
+//     (68, not 64: 16 lanes' 16-byte reads then meet distinct banks). Lane
+//     4 q + p (q < 10) reads value q's 8 words of row p, adds them, and two
+//     quad_perm adds leave value q's 64-lane total in the quad's four lanes.
+// Why LDS: on gfx950 a DPP add, a select or a compare issues in ~4.2 cycles
+// per wave and SIMD, a plain add, multiply or FMA in ~2.4, a permlane swap in
+// ~8.1 (measured, independent chains, 8 waves per SIMD), and the raster's LDS
+// pipe is mostly idle. Step 1 as DPP and the rest in LDS costs ~67 issue
+// cycles per visit; the lane-exchange network it replaces (DPP row halvings
+// per visit, then selects, quad_perms and swaps per pair of visits) ~110.
+// Leaving step 1 to LDS as well would take half as many cycles again, but
+// would fill the LDS pipe. The matrix cores don't help: an MFMA holds the
+// SIMD's vector issue for its whole time (16-32 cycles) here.
+// The reads of a visit's words are issued one visit later, before that
+// visit's arithmetic, which hides their latency; LDS serves a wave's
+// operations in order, so they precede the later visit's writes.
+// The asm block starts with two wait states for the DPP read of a value that
+// the previous VALU instruction wrote. Every step runs with all 64 lanes
+// active (every branch of the visit loop is wave-uniform, and every wave of a
+// block is full): a DPP add whose source lane were inactive would leave its
+// output unwritten.
 template <int kCtrl>
 __device__ __forceinline__ uint32_t dpp(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xf, 0xf, false);
@@ -370,149 +419,78 @@ __device__ __forceinline__ uint32_t as_u(T v) { return __builtin_bit_cast(uint32
 template <typename T>
 __device__ __forceinline__ T from_u(uint32_t v) { return __builtin_bit_cast(T, v); }
 
-template <typename T, int N, bool k32>
-__device__ __forceinline__ void swap_halve(const T* v, T* out) {
-  constexpr int H = (N + 1) / 2;
-#pragma unroll
-  for (int i = 0; i < H; i++) {
-    const uint32_t lo = as_u(v[i]);
-    const uint32_t hi = i + H < N ? as_u(v[i + H]) : as_u((T)0);
-    uint32_t a, bq;
-    if (k32) {
-      const auto r = __builtin_amdgcn_permlane32_swap(lo, hi, false, false);
-      a = r[0];
-      bq = r[1];
-    } else {
-      const auto r = __builtin_amdgcn_permlane16_swap(lo, hi, false, false);
-      a = r[0];
-      bq = r[1];
-    }
-    out[i] = from_u<T>(a) + from_u<T>(bq);
-  }
-}
+#define GS_DPP_M(OP, O, LO, HI) \
+  OP " " O ", " LO ", " LO " row_mirror row_mask:0xf bank_mask:0x3\n\t" \
+  OP " " O ", " HI ", " HI " row_mirror row_mask:0xf bank_mask:0xc\n\t"
+#define GS_ROW_STEP(OP)                \
+  "s_nop 1\n\t"                       \
+  GS_DPP_M(OP, "%0", "%5", "%10")      \
+  GS_DPP_M(OP, "%1", "%6", "%11")      \
+  GS_DPP_M(OP, "%2", "%7", "%12")      \
+  GS_DPP_M(OP, "%3", "%8", "%13")      \
+  GS_DPP_M(OP, "%4", "%9", "%14")
 
-template <typename T, int N, int kCtrl>
-__device__ __forceinline__ void dpp_halve(const T* v, T* out, bool upper) {
-  constexpr int H = (N + 1) / 2;
-#pragma unroll
-  for (int i = 0; i < H; i++) {
-    const T lo = v[i];
-    const T hi = i + H < N ? v[i + H] : (T)0;
-    const T keep = upper ? hi : lo;
-    const T send = upper ? lo : hi;
-    out[i] = keep + from_u<T>(dpp<kCtrl>(as_u(send)));
-  }
-}
-
-// Row step 1 (l ^ 15) on one visit's 10 values: lanes 0-7 of each row keep
-// values 0-4, lanes 8-15 values 5-9.
-#define GS_DPP_M(OP, O, LO, HI, CTRL, MLO, MHI) \
-  OP " " O ", " LO ", " LO " " CTRL " row_mask:0xf bank_mask:" MLO "\n\t" \
-  OP " " O ", " HI ", " HI " " CTRL " row_mask:0xf bank_mask:" MHI "\n\t"
-#define GS_ROW_STEP1(OP)                                              \
-  "s_nop 1\n\t"                                                      \
-  GS_DPP_M(OP, "%0", "%5", "%10", "row_mirror", "0x3", "0xc")         \
-  GS_DPP_M(OP, "%1", "%6", "%11", "row_mirror", "0x3", "0xc")         \
-  GS_DPP_M(OP, "%2", "%7", "%12", "row_mirror", "0x3", "0xc")         \
-  GS_DPP_M(OP, "%3", "%8", "%13", "row_mirror", "0x3", "0xc")         \
-  GS_DPP_M(OP, "%4", "%9", "%14", "row_mirror", "0x3", "0xc")         \
-  "s_nop 1"
-// Row step 2 (l ^ 7) on 5 values: lanes 0-3 and 8-11 keep values 0-2,
-// lanes 4-7 and 12-15 values 3, 4 and a zero.
-#define GS_ROW_STEP2(OP)                                              \
-  "s_nop 1\n\t"                                                      \
-  GS_DPP_M(OP, "%0", "%3", "%6", "row_half_mirror", "0x5", "0xa")     \
-  GS_DPP_M(OP, "%1", "%4", "%7", "row_half_mirror", "0x5", "0xa")     \
-  "v_mov_b32 %2, 0\n\t"                                              \
-  OP " %2, %5, %5 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"    \
-  "s_nop 1"
-
+// step 1
 template <typename T>
-__device__ __forceinline__ void visit_halve(const T* v, T* h3) {
+__device__ __forceinline__ void row_halve(const T* v, T* h5) {
   static_assert(sizeof(T) == 4, "32-bit terms");
-  T h5[5];
   if constexpr (std::is_same<T, float>::value) {
-    asm volatile(GS_ROW_STEP1("v_add_f32_dpp")
+    asm volatile(GS_ROW_STEP("v_add_f32_dpp")
                  : "=&v"(h5[0]), "=&v"(h5[1]), "=&v"(h5[2]), "=&v"(h5[3]), "=&v"(h5[4])
                  : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]),
                    "v"(v[5]), "v"(v[6]), "v"(v[7]), "v"(v[8]), "v"(v[9]));
-    asm volatile(GS_ROW_STEP2("v_add_f32_dpp")
-                 : "=&v"(h3[0]), "=&v"(h3[1]), "=&v"(h3[2])
-                 : "v"(h5[0]), "v"(h5[1]), "v"(h5[2]), "v"(h5[3]), "v"(h5[4]));
   } else {
-    asm volatile(GS_ROW_STEP1("v_add_u32_dpp")
+    asm volatile(GS_ROW_STEP("v_add_u32_dpp")
                  : "=&v"(h5[0]), "=&v"(h5[1]), "=&v"(h5[2]), "=&v"(h5[3]), "=&v"(h5[4])
                  : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]),
                    "v"(v[5]), "v"(v[6]), "v"(v[7]), "v"(v[8]), "v"(v[9]));
-    asm volatile(GS_ROW_STEP2("v_add_u32_dpp")
-                 : "=&v"(h3[0]), "=&v"(h3[1]), "=&v"(h3[2])
-                 : "v"(h5[0]), "v"(h5[1]), "v"(h5[2]), "v"(h5[3]), "v"(h5[4]));
   }
 }
-#undef GS_ROW_STEP2
-#undef GS_ROW_STEP1
+#undef GS_ROW_STEP
 #undef GS_DPP_M
 
-// The last four steps on two visits' row-halved values (the waiting one's
-// in p, the new one's in h): 20 wave totals, slots 0-9 the waiting visit's.
+// A wave's reduction scratch (5 rows of 64 words at red): where lane l writes
+// and reads, and the slot of the accumulator row it adds to (lane 4 q: q).
 template <typename T>
-__device__ __forceinline__ T pair_reduce(const T* p, const T* h) {
-  const uint32_t lane = __lane_id();
-  const T v[6] = {p[0], p[1], p[2], h[0], h[1], h[2]};
-  T c[3], d[2], e[1], g[1];
-  dpp_halve<T, 6, 0x4E>(v, c, (lane & 2) != 0);
-  dpp_halve<T, 3, 0xB1>(c, d, (lane & 1) != 0);
-  swap_halve<T, 2, false>(d, e);
-  swap_halve<T, 1, true>(e, g);
-  return g[0];
-}
-
-// The last four steps on one visit's row-halved values (a visit left
-// without a partner at the end of the tile).
-template <typename T>
-__device__ __forceinline__ T single_reduce(const T* h) {
-  const uint32_t lane = __lane_id();
-  T d[2], e[1], f[1], g[1];
-  dpp_halve<T, 3, 0x4E>(h, d, (lane & 2) != 0);
-  dpp_halve<T, 2, 0xB1>(d, e, (lane & 1) != 0);
-  swap_halve<T, 1, false>(e, f);
-  swap_halve<T, 1, true>(f, g);
-  return g[0];
-}
-
-// slot whose 64-lane total this lane holds after pair_reduce (0-9: the
-// waiting visit's terms, 10-19: the new visit's; -1: none)
-__device__ __forceinline__ int pair_slot() {
-  uint32_t va[10], vb[10], ha[3], hb[3];
-#pragma unroll
-  for (int i = 0; i < 10; i++) {
-    va[i] = (uint32_t)(i + 1);
-    vb[i] = (uint32_t)(i + 11);
+struct WaveRed {
+  T* wr;
+  const T* rd;
+  int slot;        // this lane's quad's value, clamped to 9
+  bool flusher;    // lane 4 q, q < 10
+  __device__ __forceinline__ WaveRed(float4* red, int lane) {
+    const int q = lane >> 2, qc = q < 10 ? q : 9;
+    wr = reinterpret_cast<T*>(red) + lane;
+    rd = reinterpret_cast<const T*>(red) + kRedStride * (qc % 5) + 16 * (lane & 3) + 8 * (qc / 5);
+    slot = qc;
+    flusher = q < 10 && (lane & 3) == 0;
   }
-  visit_halve<uint32_t>(va, ha);
-  visit_halve<uint32_t>(vb, hb);
-  const int s = (int)(pair_reduce<uint32_t>(ha, hb) / 64u) - 1;
-  return s >= 0 && s < 20 ? s : -1;
-}
-
-// slot whose 64-lane total this lane holds after single_reduce (-1: none)
-__device__ __forceinline__ int single_slot() {
-  uint32_t v[10], h[3];
+  __device__ __forceinline__ void write(const T* h5) const {
 #pragma unroll
-  for (int i = 0; i < 10; i++) v[i] = (uint32_t)(i + 1);
-  visit_halve<uint32_t>(v, h);
-  const int s = (int)(single_reduce<uint32_t>(h) / 64u) - 1;
-  return s >= 0 && s < 10 ? s : -1;
-}
+    for (int i = 0; i < 5; i++) wr[kRedStride * i] = h5[i];
+  }
+  __device__ __forceinline__ void read(T* w8) const {
+    const uint4 a = reinterpret_cast<const uint4*>(rd)[0], b = reinterpret_cast<const uint4*>(rd)[1];
+    w8[0] = from_u<T>(a.x); w8[1] = from_u<T>(a.y); w8[2] = from_u<T>(a.z); w8[3] = from_u<T>(a.w);
+    w8[4] = from_u<T>(b.x); w8[5] = from_u<T>(b.y); w8[6] = from_u<T>(b.z); w8[7] = from_u<T>(b.w);
+  }
+  // the 64-lane total of this lane's slot, from its quad's words
+  __device__ __forceinline__ T total(const T* w8) const {
+    T s = ((w8[0] + w8[1]) + (w8[2] + w8[3])) + ((w8[4] + w8[5]) + (w8[6] + w8[7]));
+    s = s + from_u<T>(dpp<0xB1>(as_u(s)));
+    return s + from_u<T>(dpp<0x4E>(as_u(s)));
+  }
+};
 
-// Adds one wave total to slot q of Gaussian g's accumulator row (the lanes
-// holding a total; zeros skipped).
+// Adds a visit's wave totals to Gaussian g's accumulator row (the flushing
+// lanes; zeros skipped). The asm keeps the total's last add ahead of the
+// branch, where it stays one DPP add.
 template <int kAccum, typename T>
-__device__ __forceinline__ void flush_sum(void* accum, uint32_t g, int q, T r, bool flusher) {
+__device__ __forceinline__ void flush_sum(void* accum, uint32_t g, int slot, T r, bool flusher) {
+  asm volatile("" : "+v"(r));
   if constexpr (kAccum == 0) {
-    if (flusher && r != 0u) atomicAdd((uint32_t*)accum + (int64_t)g * 12 + q, r);
+    if (flusher && r != 0u) atomicAdd((uint32_t*)accum + (int64_t)g * 12 + slot, r);
   } else {
-    if (flusher && r != 0.0f) unsafeAtomicAdd((float*)accum + (int64_t)g * 12 + q, r);
+    if (flusher && r != 0.0f) unsafeAtomicAdd((float*)accum + (int64_t)g * 12 + slot, r);
   }
 }
 
@@ -524,15 +502,14 @@ __device__ __forceinline__ void flush_sum(void* accum, uint32_t g, int q, T r, b
 template <class S, int kAccum, bool kClampColour>
 __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, const RasterBufs& b, void* accum,
                                                 int tile, float4* lds, const PixelState* in = nullptr) {
-  // four 16-byte records per staged splat, all at index j: one LDS address
+  // three 16-byte records per staged splat, all at one index: one LDS address
   float4* const sA = lds;              // mx, my, A, B
-  float4* const sB = lds + S::B;       // C, opa*comp, L, 0
+  float4* const sB = lds + S::B;       // C, opa*comp, -0.5 cnorm, id (bits)
   float4* const sC = lds + 2 * S::B;   // r, g, b, opa
-  float4* const sD = lds + 3 * S::B;   // -0.5 cnorm, 1 - opa, id (bits), 0
-  uint64_t (*const sMask)[S::kMasks] = reinterpret_cast<uint64_t (*)[S::kMasks]>(lds + 4 * S::B);
+  float4* const sRed = lds + 3 * S::B;
+  uint64_t (*const sMask)[S::kWaves] = reinterpret_cast<uint64_t (*)[S::kWaves]>(sRed + RasterLds<S>::kRed);
   uint32_t& sEnd = *reinterpret_cast<uint32_t*>(&sMask[S::kChunks][0]);
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-  const int mslot = S::mask_slot(wv);
   const PixelMap pm = pixel_of_thread<S>(cam, tile, tid);
   const int x = pm.x, y = pm.y;
   const bool inside = x < cam.W && y < cam.H;
@@ -545,20 +522,16 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
   const uint2 rg = b.ranges[tile];
   const uint32_t s = __builtin_amdgcn_readfirstlane(rg.x);
   const int64_t pi = (int64_t)y * cam.W + x;
-  const int mySlot = single_slot();
-  const bool flusher = mySlot >= 0;
-  const int mySlot20 = pair_slot();
-  const bool flusher20 = mySlot20 >= 0;
-  // A visit's terms, halved twice inside each row as they are made (3
-  // values per lane), wait for the next visit's, and the two finish in one
-  // pair_reduce (slots 0-9 the waiting visit's, 10-19 the new one's); the
-  // sums are added to the accumulators in a different order than visited,
-  // which changes nothing (integer sums; f32 atomics have no fixed order
-  // anyway).
+  // The words of the last visit wait in the wave's scratch until the next
+  // visit (or the end of the tile); before the first visit they are zeros,
+  // which add nothing.
   using AccT = typename std::conditional<kAccum == 0, uint32_t, float>::type;
-  AccT pend[3];
-  uint32_t pendGid = 0;
-  bool hasPend = false;
+  const WaveRed<AccT> red(sRed + wv * (5 * kRedStride / 4), lane);
+  {
+    const AccT z[5] = {};
+    red.write(z);
+  }
+  uint32_t lastGid = 0;
   float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float Ta = 0.0f;
   uint32_t myEnd = s;
@@ -575,8 +548,6 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
       myEnd = b.end[pi];
     }
   }
-  const bool active = inside && g.w != 0.0f;
-  const uint64_t activeMask = wave_ballot(active);
   if (tid == 0) sEnd = s;
   __syncthreads();
   if (myEnd > s) atomicMax(&sEnd, myEnd);
@@ -598,143 +569,137 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
   const float gCs[3] = {gC[0] * kS, gC[1] * kS, gC[2] * kS};
   // 16384 dot(gC, S) of the colour-behind sum S, which enters only through it
   float GS = fmaf(gCs[2], cam.bg[2], fmaf(gCs[1], cam.bg[1], gCs[0] * cam.bg[0])) * Ta;
+  // batches start at multiples of S::B keys from s, as the forward's do, so
+  // that their chunks are the forward's chunks
   for (uint32_t hi = endMax; hi > s; ) {
-    const uint32_t lo = hi - s > (uint32_t)S::B ? hi - S::B : s;
+    const uint32_t lo = s + (hi - s - 1u) / S::B * S::B;
     const int n = (int)(hi - lo);
     __syncthreads();
-    for (int c = wv; c < S::kChunks; c += S::kWaves) {
-      const int j = 64 * c + lane;
-      uint32_t cover = 0;
-      if (j < n) {
-        const uint32_t v = b.ids[lo + (uint32_t)j];
-        cover = v >> kMaskShift;
-        if (cover != 0u) {
-          const uint32_t id = v & kIdMask;
-          if (b.recFmt == 0) {
-            sA[j] = b.rec[4 * id + 0];
-            sB[j] = b.rec[4 * id + 1];
-            sC[j] = b.rec[4 * id + 2];
-            const float4 d = b.rec[4 * id + 3];
-            sD[j] = make_float4(d.y, d.z, __uint_as_float(id), 0.0f);
-          } else {
-            const float4 r1 = b.rec[3 * id + 1];
-            const float4 d = b.rec[3 * id + 2];   // comp, -0.5 cnorm, 1 - opa, opa
-            sA[j] = b.rec[3 * id + 0];
-            sB[j] = r1;
-            sC[j] = record_colour(b.recFmt, r1, d.w);
-            sD[j] = make_float4(d.y, d.z, __uint_as_float(id), 0.0f);
-          }
+    for (int c = wv; c < S::kChunks && 64 * c < n; c += S::kWaves) {
+      // key 64 c + l goes to record 64 c + 63 - l, so that the walk towards the
+      // first key is an ascending one (find-first-bit on the reversed mask)
+      const int j = 64 * c + lane, r = 64 * c + 63 - lane;
+      const uint64_t* tw = b.took + took_word<S>(s, tile, ((lo - s) >> 6) + (uint32_t)c);
+      if (lane < S::kWaves) sMask[c][lane] = tw[lane];
+      uint64_t any = 0ull;   // keys that some wave of the tile took: only these are loaded
+#pragma unroll
+      for (int w = 0; w < S::kWaves; w++) any |= tw[w];
+      if (j < n && ((any >> lane) & 1ull) != 0ull) {
+        const uint32_t id = b.ids[lo + (uint32_t)j] & kIdMask;
+        if (b.recFmt == 0) {
+          const float4 r1 = b.rec[4 * id + 1];
+          sA[r] = b.rec[4 * id + 0];
+          sC[r] = b.rec[4 * id + 2];
+          sB[r] = make_float4(r1.x, r1.y, b.rec[4 * id + 3].y, __uint_as_float(id));
+        } else {
+          const float4 r1 = b.rec[3 * id + 1];
+          const float4 d = b.rec[3 * id + 2];   // comp, -0.5 cnorm, 1 - opa, opa
+          sA[r] = b.rec[3 * id + 0];
+          sC[r] = record_colour(b.recFmt, r1, d.w);
+          sB[r] = make_float4(r1.x, r1.y, d.y, __uint_as_float(id));
         }
       }
-      store_masks<S>(cover, sMask[c]);
     }
     __syncthreads();
     for (int c = S::kChunks - 1; c >= 0; c--) {
-      uint64_t m = uniform64(sMask[c][mslot]);
       const uint32_t g0 = lo + 64u * (uint32_t)c;   // key of bit 0
-      if (waveEnd <= g0) m = 0ull;
-      else if (waveEnd - g0 < 64u) m &= (1ull << (waveEnd - g0)) - 1ull;
+      if (waveEnd <= g0) continue;                  // no lane got this far: the words may be stale
+      uint64_t m = uniform64(sMask[c][wv]);
+      if (waveEnd - g0 < 64u) m &= (1ull << (waveEnd - g0)) - 1ull;
+      m = __builtin_bitreverse64(m);
+      // record r of the chunk is key g0 + 63 - r: before this lane's end when
+      // r is above pastEnd
+      const int pastEnd = (int)(g0 + 63u - myEnd);
       while (m) {
-        const int bit = 63 - (int)__builtin_clzll(m);
-        m &= ~(1ull << bit);
-        const int j = c * 64 + bit;
-        const uint32_t k = lo + (uint32_t)j;
+        const int bit = (int)__builtin_ctzll(m);
+        clear_bit(m, bit);
         // Straight-line for all 64 lanes; lanes that do not take the splat
         // (outside the image, past their `end`, outside the cutoff, alpha
-        // below A_MIN) keep their state and contribute zero terms. The wave
-        // leaves as soon as no lane is inside the cutoff (before the exp) or
-        // no lane takes the splat.
-        const uint32_t jo = lds_offset((uint32_t)j * 16u);
-        const float4 a = lds_at<float4>(sA, jo);
-        const float2 bb = lds_at<float2>(sB, jo);   // C, opa*comp
-        // keep both in this one 8-byte read (otherwise the compiler sinks
-        // the second word into the next block with its own address move)
-        asm volatile("" ::"v"(bb.y));
+        // below A_MIN) keep their state and contribute zero terms. Some
+        // lane took the splat in the forward, so there is nothing to vote on.
+        AccT w8[8];
+        red.read(w8);   // the previous visit's words
+        const uint32_t jo = lds_offset((uint32_t)bit * 16u);
+        const float4 a = lds_at<float4>(sA + 64 * c, jo);
+        const float4 bb = lds_at<float4>(sB + 64 * c, jo);   // C, opa*comp, -0.5 cnorm, id
         const float dx = px - a.x, dy = py - a.y;
         const float cA = a.z, cB = a.w, cC = bb.x;
         const float t2 = fmaf(cC * dy, dy, (cA * dx) * dx);
         // clamped to [0, 87] as in the forward pass
         const float e = clamp_e(fmaf(0.5f, t2, (cB * dx) * dy));
-        // votes of single compares, combined in scalar registers (a vote
-        // of a combined condition costs two VALU instructions)
-        const bool live = active && k < myEnd && e <= cut.eCut;
-        const uint64_t liveMask = activeMask & wave_ballot(k < myEnd) & wave_ballot(e <= cut.eCut);
-        if (liveMask == 0ull) continue;
         const float G = gs_expf_raster(-e);
         const float araw = bb.y * G;
         const float alpha = fminf(0.99f, araw);
-        const bool contrib = live && alpha >= cut.aMin;
-        if ((liveMask & wave_ballot(alpha >= cut.aMin)) == 0ull) continue;
+        const bool contrib = bit > pastEnd && e <= cut.eCut && alpha >= cut.aMin;
+        const float4 c4 = lds_at<float4>(sC + 64 * c, jo);
+        // Tb = Ta / (1 - alpha), S / (1 - alpha) through one reciprocal.
+        // 1 - alpha lies in [0.0099, 1] (alpha in [0, 0.99]); on [2^-9, 1]
+        // v_rcp_f32 refined by one FMA Newton step equals the correctly
+        // rounded 1/x for every float (checked exhaustively on gfx950). A
+        // lane that does not take the splat has alpha 0 here: its reciprocal
+        // is exactly 1, so Tb = Ta and aT = 0 without a select each.
+        const float alphaE = contrib ? alpha : 0.0f;
+        const float rom = rcp_exact_unit(1.0f - alphaE);
+        const float Tb = Ta * rom;
+        const float gcol = fmaf(gCs[2], c4.z, fmaf(gCs[1], c4.y, gCs[0] * c4.x));   // scaled
+        // Every term is a product with galpha or aT, which are zero for the
+        // lanes that do not take the splat (all other factors are finite).
+        const float galphaS = (contrib && !(araw > 0.99f)) ? fmaf(gcol, Tb, -(GS * rom)) : 0.0f;
+        const float aT = alphaE * Tb;
+        const float ga = galphaS * araw;
+        const float gq = ga * bb.z;
+        const float gqdx = gq * dx;
         float v[10];
-        uint32_t gid;
-        {
-          const float4 c4 = lds_at<float4>(sC, jo);
-          const float4 d2 = lds_at<float4>(sD, jo);   // -0.5 cnorm, 1 - opa, id
-          asm volatile("" ::"v"(d2.z));
-          gid = __float_as_uint(d2.z);
-          // Tb = Ta / (1 - alpha), S / (1 - alpha) through one reciprocal.
-          // 1 - alpha lies in [0.0099, 1] (alpha in [0, 0.99]); on [2^-9, 1]
-          // v_rcp_f32 refined by one FMA Newton step equals the correctly
-          // rounded 1/x for every float (checked exhaustively on gfx950).
-          const float rom = rcp_exact_unit(1.0f - alpha);
-          const float Tb = Ta * rom;
-          const float gcol = fmaf(gCs[2], c4.z, fmaf(gCs[1], c4.y, gCs[0] * c4.x));   // scaled
-          // Every term is a product with galpha or aT; zeroing those two for
-          // the lanes that do not take the splat zeroes all ten terms (all
-          // other factors are finite), and leaves the taking lanes' bits as is.
-          const float galphaS = (contrib && !(araw > 0.99f)) ? fmaf(gcol, Tb, -(GS * rom)) : 0.0f;
-          const float aT = contrib ? alpha * Tb : 0.0f;
-          const float ga = galphaS * araw;
-          const float gq = ga * d2.x;
-          const float gqdx = gq * dx;
-          v[0] = ga * (cA * dx + cB * dy);
-          v[1] = ga * (cB * dx + cC * dy);
-          v[2] = gqdx * dx;
-          v[3] = 2.0f * (gqdx * dy);        // the middle conic term is 2 gq dx dy
-          v[4] = (gq * dy) * dy;
-          v[5] = galphaS * c4.w * G;
-          v[6] = ga * d2.y;
-          v[7] = gCs[0] * aT;
-          v[8] = gCs[1] * aT;
-          v[9] = gCs[2] * aT;
-          GS = fmaf(gcol, aT, GS);
-          Ta = contrib ? Tb : Ta;
-        }
+        v[0] = ga * (cA * dx + cB * dy);
+        v[1] = ga * (cB * dx + cC * dy);
+        v[2] = gqdx * dx;
+        v[3] = 2.0f * (gqdx * dy);        // the middle conic term is 2 gq dx dy
+        v[4] = (gq * dy) * dy;
+        v[5] = galphaS * c4.w * G;
+        v[6] = ga * (1.0f - c4.w);
+        v[7] = gCs[0] * aT;
+        v[8] = gCs[1] * aT;
+        v[9] = gCs[2] * aT;
+        GS = fmaf(gcol, aT, GS);
+        Ta = Tb;
         AccT cur[10];
         if constexpr (kAccum == 0) {
-          // i32(clamp(v * 16384, -1e9, 1e9)) per pixel; v already carries the scale
+          // i32(clamp(v * 16384, -1e9, 1e9)) per pixel; v already carries the
+          // scale. Terms beyond the clamp are rare, so one test of the largest
+          // magnitude stands for the clamps of the seven terms that carry
+          // galpha (they are NaN together, and then so is the maximum; a NaN
+          // converts to the lower clamp).
+          const float m = max3abs(max3abs(max3abs(v[0], v[1], v[2]), v[3], v[4]), v[5], v[6]);
+          if (wave_ballot(!(m <= 1.0e9f)) != 0ull) {
+#pragma unroll
+            for (int q = 0; q < 7; q++) v[q] = fminf(fmaxf(v[q], -1.0e9f), 1.0e9f);
+          }
 #pragma unroll
           for (int q = 0; q < 10; q++)
-            cur[q] = (q >= 7 && !kClampColour) ? (uint32_t)(int32_t)v[q]
-                                                : (uint32_t)(int32_t)fminf(fmaxf(v[q], -1.0e9f), 1.0e9f);
+            cur[q] = (q >= 7 && kClampColour) ? (uint32_t)(int32_t)fminf(fmaxf(v[q], -1.0e9f), 1.0e9f)
+                                               : (uint32_t)(int32_t)v[q];
         } else {
 #pragma unroll
           for (int q = 0; q < 10; q++) cur[q] = v[q];
         }
-        AccT h[3];
-        visit_halve<AccT>(cur, h);
-        if (hasPend) {
-          const AccT r = pair_reduce<AccT>(pend, h);
-          const uint32_t g2 = mySlot20 < 10 ? pendGid : gid;
-          flush_sum<kAccum>(accum, g2, mySlot20 % 10, r, flusher20);
-        }
-        // copied on both paths (after a pair it is never read), so the
-        // waiting values need no merge of two register sets at the join
-#pragma unroll
-        for (int q = 0; q < 3; q++) pend[q] = h[q];
-        pendGid = gid;
-        hasPend = !hasPend;
+        AccT h[5];
+        row_halve<AccT>(cur, h);
+        flush_sum<kAccum>(accum, lastGid, red.slot, red.total(w8), red.flusher);
+        red.write(h);
+        lastGid = __float_as_uint(bb.w);
       }
     }
     hi = lo;
   }
-  if (hasPend) flush_sum<kAccum>(accum, pendGid, mySlot, single_reduce<AccT>(pend), flusher);
+  AccT w8[8];
+  red.read(w8);
+  flush_sum<kAccum>(accum, lastGid, red.slot, red.total(w8), red.flusher);
 }
 
 template <class S, int kLoss>
 __global__ __launch_bounds__(S::kThreads) void k_raster_fwd(Cam cam, Cut cut, RasterBufs b) {
   __shared__ float4 lds[RasterLds<S>::kFwd];
-  raster_fwd_tile<S, kLoss>(cam, cut, b, tile_of_block(b), lds);
+  raster_fwd_tile<S, kLoss, kLoss == 2>(cam, cut, b, tile_of_block(b), lds);
 }
 
 template <class S, int kAccum, bool kClampColour>
@@ -753,7 +718,7 @@ __global__ __launch_bounds__(S::kThreads) void k_raster_fwd_bwd(Cam cam, Cut cut
   __shared__ float4 lds[RasterLds<S>::kBoth];   // the two passes' layouts share it
   const int tile = tile_of_block(b);
   PixelState ps;
-  raster_fwd_tile<S, 1>(cam, cut, b, tile, lds, &ps);
+  raster_fwd_tile<S, 1, true>(cam, cut, b, tile, lds, &ps);
   __syncthreads();   // the forward's last LDS reads are done
   raster_bwd_tile<S, kAccum, kClampColour>(cam, cut, b, accum, tile, lds, &ps);
 }
@@ -801,7 +766,7 @@ k_raster_fwd_bwd_views(const ViewBlock* __restrict__ vb, Cut cut, uint32_t* queu
     const Cam& cam = vb->cams[it.v];
     const RasterBufs& b = vb->bufs[it.v];
     PixelState ps;
-    raster_fwd_tile<S, 1>(cam, cut, b, it.tile, lds, &ps);
+    raster_fwd_tile<S, 1, true>(cam, cut, b, it.tile, lds, &ps);
     __syncthreads();   // the forward's last LDS reads are done
     raster_bwd_tile<S, kAccum, kClampColour>(cam, cut, b, gs_global(vb->accum[it.v]), it.tile, lds, &ps);
   }
@@ -817,7 +782,7 @@ __global__ __launch_bounds__(S::kThreads) void k_raster_fwd_bwd_view(const ViewB
   __shared__ float4 lds[RasterLds<S>::kBoth];
   const int tile = tile_of_block(b);
   PixelState ps;
-  raster_fwd_tile<S, 1>(cam, cut, b, tile, lds, &ps);
+  raster_fwd_tile<S, 1, true>(cam, cut, b, tile, lds, &ps);
   __syncthreads();
   raster_bwd_tile<S, kAccum, kClampColour>(cam, cut, b, gs_global(vb->accum[v]), tile, lds, &ps);
 }
@@ -835,6 +800,17 @@ static void with_shape(const RasterShape& sh, F&& f) {
   if (sh.tile == 8) with_batch<8>(sh.batch, f);
   else if (sh.tile == 32) with_batch<32>(sh.batch, f);
   else with_batch<16>(sh.batch, f);
+}
+
+size_t raster_took_bytes(int w, int h, int64_t keys) {
+  // took_word's last row at each tile size: one word per wave (tile^2 / 64)
+  size_t words = 0;
+  for (int t = 8; t <= 32; t *= 2) {
+    const size_t tiles = (size_t)((w + t - 1) / t) * (size_t)((h + t - 1) / t);
+    const size_t need = ((size_t)keys / 64 + tiles + 1) * (size_t)(t * t / 64);
+    words = words > need ? words : need;
+  }
+  return words * 8;
 }
 
 bool raster_shape_ok(int tile, int batch) {

@@ -115,6 +115,7 @@ struct gs_trainer {
   float* Tfin = nullptr;
   uint32_t* endIdx = nullptr;
   float4* gC = nullptr;
+  uint64_t* took = nullptr;      // the training forward's taken keys per wave (RasterBufs::took)
   float* ssimScratch = nullptr;  // 9 x maxPix SSIM partials (L1 + D-SSIM loss only)
   uint32_t* targets = nullptr;
   int64_t totalPx = 0;
@@ -148,7 +149,7 @@ struct gs_trainer {
   // buffers; slot 0 is the single-view set above
   struct ViewSlot {
     float4* rec; uint32_t* cnt; void* accum; uint32_t* ids; uint2* ranges; uint32_t* tileOrder;
-    float4* img; float* T; uint32_t* end; float4* gC;
+    float4* img; float* T; uint32_t* end; float4* gC; uint64_t* took;
     // the batched binning's own copies (slot 0: the single-view buffers)
     uint32_t* depthKey; uint2* rect; uint32_t* chunkKeys; uint32_t* blockStart; uint32_t* table;
     uint32_t* visPart; uint32_t* tileCnt; uint64_t* keys; uint64_t* tmp; uint64_t* totalKeys;
@@ -496,6 +497,7 @@ int run_raster(gs_trainer* h, const Cam& cam, int loss, double* statsBuf, bool w
   b.T = h->Tfin;
   b.end = h->endIdx;
   b.gC = h->gC;
+  b.took = h->took;
   b.tgt = h->targets;
   b.stats = statsBuf;
   if (withBwd) {
@@ -729,6 +731,7 @@ int step_impl(gs_trainer* h, int ci, gs_debug_out* dbg) {
   b.T = h->Tfin;
   b.end = h->endIdx;
   b.gC = h->gC;
+  b.took = h->took;
   if (ssim) {
     Scope s(h, "raster_bwd", 0.0);
     launch_raster_bwd(h->st, h->shape, cam, make_cut(h), b, h->o.gradAccum, h->accum, false);
@@ -989,6 +992,7 @@ int fill_views(gs_trainer* h, const int* ci, int count, int activeDeg, double* s
     b.T = sl.T;
     b.end = sl.end;
     b.gC = sl.gC;
+    b.took = sl.took;
     b.tgt = h->targets;
     b.stats = statsBuf;
     vb.accum[k] = sl.accum;
@@ -1369,6 +1373,9 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
   rc |= dalloc(h, &h->Tfin, (size_t)h->maxPix * 4);
   rc |= dalloc(h, &h->endIdx, (size_t)h->maxPix * 4);
   rc |= dalloc(h, &h->gC, (size_t)h->maxPix * 16);
+  size_t tookBytes = 0;
+  for (const CamMeta& m : h->cams) tookBytes = std::max(tookBytes, raster_took_bytes(m.c.w, m.c.h, h->entriesCap));
+  rc |= dalloc(h, &h->took, tookBytes);
   if (h->o.loss == GS_LOSS_L1_DSSIM) rc |= dalloc(h, &h->ssimScratch, (size_t)h->maxPix * 36);
   rc |= dalloc(h, &h->targets, tgt.size() * 4);
   rc |= dalloc(h, &h->stats, 32);
@@ -1377,7 +1384,7 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
   // batched views: slot 0 is the single-view set, slots 1.. their own copies
   h->vslots.assign((size_t)h->o.viewsPerStep, gs_trainer::ViewSlot{});
   h->vslots[0] = {h->rec, h->cnt, h->accum, h->tvA, h->ranges, h->tileOrder, h->img, h->Tfin, h->endIdx, h->gC,
-                  h->depthKey, h->rect, h->sort.chunkKeys, h->sort.blockStart, h->sort.segTable, h->sort.visPart,
+                  h->took, h->depthKey, h->rect, h->sort.chunkKeys, h->sort.blockStart, h->sort.segTable, h->sort.visPart,
                   h->sort.tileCnt, (uint64_t*)h->tkA, (uint64_t*)h->tkB, h->totalKeys};
   for (size_t k = 1; k < h->vslots.size(); k++) {
     gs_trainer::ViewSlot& v = h->vslots[k];
@@ -1391,6 +1398,7 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
     rc |= dalloc(h, &v.T, (size_t)h->maxPix * 4);
     rc |= dalloc(h, &v.end, (size_t)h->maxPix * 4);
     rc |= dalloc(h, &v.gC, (size_t)h->maxPix * 16);
+    rc |= dalloc(h, &v.took, tookBytes);
   }
   if (h->o.viewsPerStep > 1) {
     rc |= dalloc(h, &h->dVB, sizeof(ViewBlock));
@@ -1544,6 +1552,7 @@ int tune_pass(gs_trainer* h, const int* ci, int count, int activeDeg) {
     b.T = h->Tfin;
     b.end = h->endIdx;
     b.gC = h->gC;
+    b.took = h->took;
     launch_raster_bwd(h->st, h->shape, cam, make_cut(h), b, h->o.gradAccum, h->accum, false);
     HIPCK(hipGetLastError());
     return GS_OK;

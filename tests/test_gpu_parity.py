@@ -515,3 +515,15 @@ def test_l1_dssim_training_reduces_loss():
     last = t.readLoss()
     t.destroy()
     assert last < first
+
+
+@pytest.mark.parametrize("gain", [6.0e4, 1.0e6])
+def test_gradient_terms_beyond_the_fixed_point_clamp(gain):
+    """An exposure gain of 6e4 brings single pixels' x16384 gradient terms
+    past the +-1e9 clamp (the largest gain whose colour terms need none), one
+    of 1e6 the colour terms too: sums and updates stay bit-exact."""
+    print(f"gain {gain}", flush=True)
+    params, sh, cams, images, W, H, radius, opts = rig_setup(3)
+    # the camera struct holds the log gain in f32
+    cams = [dict(c, g=float(np.float32(math.log(gain)))) for c in cams]
+    _run_pair(params, sh, cams, images, W, H, radius, opts, 3, steps=2, start_iter=5000)
