@@ -204,6 +204,42 @@ def test_sort_strategies_give_the_same_permutation():
         np.testing.assert_array_equal(a["img"], b["img"])
 
 
+@pytest.mark.parametrize("depths", ["random", "equal", "clustered"])
+@pytest.mark.parametrize("n", [1024, 1025, 1537, 4099, 65537, 150000])
+def test_one_long_tile_segment_sorts_as_the_radix_strategy(n, depths):
+    """A one-tile view under n splats: one segment of n keys, at the last
+    size sorted in one piece, the first sizes that split into three, four
+    and nine buckets, and the sizes past the 128 buckets, whose larger
+    buckets are merged. Equal depths order by id; clustered ones put nine
+    keys in ten within 1% of the depth range, in stretches of the input, so
+    that the sampled splitters are uneven. Keys, ids and image are those of
+    the depth-then-tile radix strategy."""
+    rng = np.random.default_rng(n)
+    p = np.zeros((n, 16), np.float32)
+    z = {"random": rng.uniform(1.0, 9.0, n), "equal": np.full(n, 3.0),
+         "clustered": np.where(np.arange(n) // 64 % 10 == 0, rng.uniform(1.0, 9.0, n), rng.uniform(3.0, 3.08, n))}[depths]
+    p[:, 0:2] = rng.uniform(-0.3, 0.3, (n, 2)) * z[:, None]
+    p[:, 2] = z
+    p[:, 3:6] = np.log(0.2 * z)[:, None]
+    p[:, 6] = 1.0
+    p[:, 10:13] = rng.normal(0, 1, (n, 3))
+    p[:, 13] = rng.uniform(-3, 2, n)
+    W = H = 16
+    cams = [{"imgIdx": 0, "R": [1, 0, 0, 0, 1, 0, 0, 0, 1], "t": [0, 0, 0], "f": 16.0, "cx": 8, "cy": 8, "w": W, "h": H}]
+    images = [{"tw": W, "th": H, "rgb": np.full((W * H, 3), 0.5, np.float32)}]
+    outs = []
+    for mode in (gsabi.GS_SORT_TILE_SEGMENTS, gsabi.GS_SORT_DEPTH_THEN_TILE):
+        t = _trainer(p, None, cams, images, W, H, 1.0, {}, shDeg=0, sortMode=mode)
+        outs.append(t.step_debug(0, want=("ids", "keys", "tileRanges", "img")))
+        t.destroy()
+    a, b = outs
+    assert a["numKeys"] == b["numKeys"] == n
+    np.testing.assert_array_equal(a["keys"], b["keys"])
+    np.testing.assert_array_equal(a["ids"], b["ids"])
+    np.testing.assert_array_equal(a["tileRanges"], b["tileRanges"])
+    np.testing.assert_array_equal(a["img"].view(np.uint32), b["img"].view(np.uint32))
+
+
 def test_views_above_the_segment_tile_limit_fall_back_to_radix():
     """A 2112x2112 view has 17424 tiles, above the 16384 the tile-segment
     scan handles: the default sort falls back to depth-then-tile and gives
