@@ -96,7 +96,7 @@ GS_HD gs_cover_splat gs_cover_prepare(float mx, float my, float A, float B, floa
 // conic that is not positive definite keeps every block: kA = kC = 0 there
 // and the mask computed for it is discarded).
 GS_HD uint32_t gs_cover_tile_mask(const gs_cover_splat* s, int tx, int ty, int T) {
-  const float x0 = (float)(tx * T) + 0.5f, y0 = (float)(ty * T) + 0.5f;
+  const float x0 = (float)tx * (float)T + 0.5f, y0 = (float)ty * (float)T + 0.5f;   // exact: no integer product
   const float h1 = (float)(T / 2 - 1), h2 = (float)(T / 2), h3 = (float)(T - 1);
   const float u[4] = {x0 - s->mx, (x0 + h1) - s->mx, (x0 + h2) - s->mx, (x0 + h3) - s->mx};
   const float w[4] = {y0 - s->my, (y0 + h1) - s->my, (y0 + h2) - s->my, (y0 + h3) - s->my};

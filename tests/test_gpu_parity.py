@@ -240,6 +240,49 @@ def test_one_long_tile_segment_sorts_as_the_radix_strategy(n, depths):
     np.testing.assert_array_equal(a["img"].view(np.uint32), b["img"].view(np.uint32))
 
 
+@pytest.mark.parametrize("n,big,small", [(3000, 3000, 0.0), (530000, 1500, 0.05), (530000, 600, 0.003)],
+                         ids=["every_tile", "bands", "one_band"])
+def test_binning_of_wide_splats_as_the_radix_strategy(n, big, small):
+    """A 640x480 view (1200 tiles) whose first `big` splats cover every tile:
+    their count and scatter rounds hold 1.2M keys, walked in windows of
+    65536. At 530000 splats (256 blocks) of log-scale log(0.05) the view
+    holds more than 12 keys per block and tile, so the scatter takes the
+    tiles in bands of rows, which the splats cross; small ones stay below
+    that. A tenth of the splats are culled, in runs and singly. Keys, ids,
+    ranges and image are those of the depth-then-tile radix strategy."""
+    rng = np.random.default_rng(7)
+    W, H, f = 640, 480, 400.0
+    p = np.zeros((n, 16), np.float32)
+    z = rng.uniform(2.0, 4.0, n)
+    z[rng.random(n) < 0.05] = -1.0                          # behind the camera
+    z[n // 3:n // 3 + n // 20] = -1.0
+    p[:, 0] = rng.uniform(-0.5, 0.5, n) * W / f * z
+    p[:, 1] = rng.uniform(-0.5, 0.5, n) * H / f * z
+    p[:, 2] = z
+    p[:, 3:6] = np.log(max(small, 1e-3)) + rng.normal(0, 0.1, (n, 3))
+    p[:big, 0:2] = 0.0
+    p[:big, 3:6] = np.log(4.0)
+    p[:, 6] = 1.0
+    p[:, 10:13] = rng.normal(0, 1, (n, 3))
+    p[:, 13] = rng.uniform(-4, -1, n)
+    cams = [{"imgIdx": 0, "R": [1, 0, 0, 0, 1, 0, 0, 0, 1], "t": [0, 0, 0], "f": f, "cx": W / 2, "cy": H / 2, "w": W, "h": H}]
+    images = [{"tw": W, "th": H, "rgb": np.full((W * H, 3), 0.5, np.float32)}]
+    outs = []
+    for mode in (gsabi.GS_SORT_TILE_SEGMENTS, gsabi.GS_SORT_DEPTH_THEN_TILE):
+        t = _trainer(p, None, cams, images, W, H, 1.0, {}, shDeg=0, sortMode=mode, radClamp=2000,
+                     entriesCap=1 << 24)
+        outs.append(t.step_debug(0, want=("ids", "keys", "tileRanges", "img")))
+        t.destroy()
+    a, b = outs
+    per_run = a["numKeys"] / (min(256, -(-n // 2048)) * 1200)
+    assert a["numKeys"] == b["numKeys"] > 0.8 * big * 1200
+    assert (per_run >= 12) == (small != 0.003)
+    np.testing.assert_array_equal(a["keys"], b["keys"])
+    np.testing.assert_array_equal(a["ids"], b["ids"])
+    np.testing.assert_array_equal(a["tileRanges"], b["tileRanges"])
+    np.testing.assert_array_equal(a["img"].view(np.uint32), b["img"].view(np.uint32))
+
+
 def test_views_above_the_segment_tile_limit_fall_back_to_radix():
     """A 2112x2112 view has 17424 tiles, above the 16384 the tile-segment
     scan handles: the default sort falls back to depth-then-tile and gives
