@@ -580,6 +580,39 @@ def test_l1_dssim_loss_against_f64(tile, batch):
     np.testing.assert_array_equal(g["accum"], acc)
 
 
+@pytest.mark.parametrize("W,H", [(32, 16), (33, 17), (31, 15), (1, 1), (1, 41), (70, 5), (5, 6), (64, 49)])
+def test_l1_dssim_loss_at_the_edges_of_its_tiles(W, H):
+    """The SSIM kernels' 32x16 tiles, whole, one pixel over and one short,
+    views narrower than the window, and ragged ones; a tenth of the pixels
+    invalid. The bounds are those of the larger view above (f32 blur sums
+    against f64): 3e-4 of the largest gradient, 1e-5 relative on the loss."""
+    rng = np.random.default_rng(100 * W + H)
+    n, f = 300, 20.0
+    p = np.zeros((n, 16), np.float32)
+    z = rng.uniform(2.0, 4.0, n)
+    p[:, 0] = rng.uniform(-0.5, 0.5, n) * W / f * z
+    p[:, 1] = rng.uniform(-0.5, 0.5, n) * H / f * z
+    p[:, 2] = z
+    p[:, 3:6] = np.log(0.3)
+    p[:, 6] = 1.0
+    p[:, 10:13] = rng.normal(0, 1, (n, 3))
+    p[:, 13] = rng.uniform(-2, 1, n)
+    cams = [{"imgIdx": 0, "R": [1, 0, 0, 0, 1, 0, 0, 0, 1], "t": [0, 0, 0], "f": f, "cx": W / 2, "cy": H / 2, "w": W, "h": H}]
+    rgb = rng.random((H * W, 3)).astype(np.float32)
+    rgb[rng.random(H * W) < 0.1, 0] = -1.0
+    rgb[0] = 0.5
+    images = [{"tw": W, "th": H, "rgb": rgb}]
+    t = _trainer(p, None, cams, images, W, H, 1.0, {}, shDeg=0, loss=gsabi.GS_LOSS_L1_DSSIM, ssimLambda=0.2)
+    g = t.step_debug(0, want=("img", "gC", "stats"))
+    t.destroy()
+    st64 = O.Stage(O.make_opts(shDeg=0), "f64")
+    gC64, valid, stats64 = st64.loss_l1ssim(O.make_cam(cams[0]), g["img"].astype(np.float64), O.pack_targets(rgb), 0.2)
+    np.testing.assert_array_equal(g["gC"][:, 3] != 0, valid != 0)
+    assert not g["gC"][valid == 0].any()
+    assert np.abs(g["gC"][:, :3] - gC64).max() <= 3e-4 * np.abs(gC64).max()
+    np.testing.assert_allclose(g["stats"][:3], stats64, rtol=1e-5)
+
+
 def test_l1_dssim_training_reduces_loss():
     p, sh, cams, images, W, H, radius = config1_setup(n=8000)
     t = _trainer(p, sh, cams, images, W, H, radius, {}, shDeg=2, loss=gsabi.GS_LOSS_L1_DSSIM)
