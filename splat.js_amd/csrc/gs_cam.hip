@@ -17,7 +17,12 @@
 
 namespace gs {
 
-constexpr int kCamBlocks = 1024;
+// Few blocks of many waves: a block ends in one atomic per slot, and atomics on
+// one line go through one after another, about 14 ns each. 303k pixels and
+// 123k Gaussians: exposure 14.1 -> 5.9 us, pose 10.7 -> 9.2 against 1024
+// blocks of 256 threads.
+constexpr int kCamThreads = 1024;
+constexpr int kCamBlocks = 256;
 
 __device__ __forceinline__ uint32_t cam_fix(float v) {
   return (uint32_t)(int32_t)clampf(v * 64.0f, -1.0e9f, 1.0e9f);
@@ -32,19 +37,18 @@ __device__ __forceinline__ void cross3(const float* a, const float* b, float* c)
 // Wrapping block sum of N per-thread values; slot k goes to *dst[k].
 template <int N>
 __device__ __forceinline__ void block_add(uint32_t (&v)[N], uint32_t* const (&dst)[N]) {
-  __shared__ uint32_t part[kBlock / 64][N];
+  __shared__ uint32_t part[kCamThreads / 64][N];
 #pragma unroll
-  for (int k = 0; k < N; k++)
-    for (int o = 32; o > 0; o >>= 1) v[k] += (uint32_t)__shfl_xor((int)v[k], o);
+  for (int k = 0; k < N; k++) v[k] = wave_incl_scan(v[k]);
   const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0)
+  if ((threadIdx.x & 63) == 63)   // the wave's sums
 #pragma unroll
     for (int k = 0; k < N; k++) part[w][k] = v[k];
   __syncthreads();
   if (threadIdx.x < N) {
     uint32_t s = 0;
 #pragma unroll
-    for (int q = 0; q < kBlock / 64; q++) s += part[q][threadIdx.x];
+    for (int q = 0; q < kCamThreads / 64; q++) s += part[q][threadIdx.x];
     if (s != 0u) atomicAdd(dst[threadIdx.x], s);
   }
 }
@@ -53,11 +57,11 @@ __device__ __forceinline__ void block_add(uint32_t (&v)[N], uint32_t* const (&ds
 // stored image exactly as the forward pass evaluates them: per valid pixel
 // d/d(log gain) = dot(eg, C) * gain and d/d(bias) = eg.x + eg.y + eg.z,
 // eg = err / sqrt(err^2 + 0.03^2), err = gain * C + bias - target.
-__global__ __launch_bounds__(kBlock) void k_cam_exposure(Cam cam, const float4* __restrict__ img,
+__global__ __launch_bounds__(kCamThreads) void k_cam_exposure(Cam cam, const float4* __restrict__ img,
                                                          const uint32_t* __restrict__ tgt, uint32_t* row) {
   const int64_t npx = (int64_t)cam.W * cam.H;
   uint32_t acc[2] = {0u, 0u};
-  for (int64_t pi = (int64_t)blockIdx.x * kBlock + threadIdx.x; pi < npx; pi += (int64_t)gridDim.x * kBlock) {
+  for (int64_t pi = (int64_t)blockIdx.x * kCamThreads + threadIdx.x; pi < npx; pi += (int64_t)gridDim.x * kCamThreads) {
     const uint32_t pk = tgt[cam.tgtOffset + pi];
     if ((pk >> 24) == 0u) continue;
     const float4 o4 = img[pi];
@@ -82,9 +86,9 @@ __global__ __launch_bounds__(kBlock) void k_cam_exposure(Cam cam, const float4* 
 // dL/dlog f = f dL/df over the mean and Jacobian paths. kClear also zeroes
 // the screen-space accumulators (an evaluation pass, which runs no update).
 template <int kAccum, bool kClear>
-__global__ __launch_bounds__(kBlock) void k_cam_pose(Cam cam, CamPoseBufs b) {
+__global__ __launch_bounds__(kCamThreads) void k_cam_pose(Cam cam, CamPoseBufs b) {
   uint32_t acc[7] = {0u, 0u, 0u, 0u, 0u, 0u, 0u};
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < b.n; i += (int64_t)gridDim.x * kBlock) {
+  for (int64_t i = (int64_t)blockIdx.x * kCamThreads + threadIdx.x; i < b.n; i += (int64_t)gridDim.x * kCamThreads) {
     int4* ac = (int4*)b.accum + 3 * i;
     const int4 a0 = ac[0], a1 = ac[1];
     if (kClear) {
@@ -138,25 +142,25 @@ __global__ __launch_bounds__(kBlock) void k_cam_pose(Cam cam, CamPoseBufs b) {
 }
 
 static unsigned cam_grid(int64_t items) {
-  const int64_t g = (items + kBlock - 1) / kBlock;
+  const int64_t g = (items + kCamThreads - 1) / kCamThreads;
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>(g, kCamBlocks));
 }
 
 void launch_cam_exposure(hipStream_t st, const Cam& cam, const float4* img, const uint32_t* tgt, uint32_t* row) {
   const int64_t npx = (int64_t)cam.W * cam.H;
   if (npx <= 0) return;
-  k_cam_exposure<<<cam_grid(npx), kBlock, 0, st>>>(cam, img, tgt, row);
+  k_cam_exposure<<<cam_grid(npx), kCamThreads, 0, st>>>(cam, img, tgt, row);
 }
 
 void launch_cam_pose(hipStream_t st, int accumMode, bool clear, const Cam& cam, const CamPoseBufs& b) {
   if (b.n <= 0) return;
   const dim3 grid(cam_grid(b.n));
   if (accumMode == 0) {
-    if (clear) k_cam_pose<0, true><<<grid, kBlock, 0, st>>>(cam, b);
-    else k_cam_pose<0, false><<<grid, kBlock, 0, st>>>(cam, b);
+    if (clear) k_cam_pose<0, true><<<grid, kCamThreads, 0, st>>>(cam, b);
+    else k_cam_pose<0, false><<<grid, kCamThreads, 0, st>>>(cam, b);
   } else {
-    if (clear) k_cam_pose<1, true><<<grid, kBlock, 0, st>>>(cam, b);
-    else k_cam_pose<1, false><<<grid, kBlock, 0, st>>>(cam, b);
+    if (clear) k_cam_pose<1, true><<<grid, kCamThreads, 0, st>>>(cam, b);
+    else k_cam_pose<1, false><<<grid, kCamThreads, 0, st>>>(cam, b);
   }
 }
 

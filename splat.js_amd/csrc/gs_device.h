@@ -84,6 +84,30 @@ __device__ __forceinline__ T* gs_global(T* const& field) {
 // instructions per vote.
 __device__ __forceinline__ uint64_t wave_ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
+// x of the lane a DPP control selects, 0 where it selects none
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint32_t dpp_or0(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, kRows, 0xf, false);
+}
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint64_t dpp_or0(uint64_t x) {
+  return ((uint64_t)dpp_or0<kCtrl, kRows>((uint32_t)(x >> 32)) << 32) | dpp_or0<kCtrl, kRows>((uint32_t)x);
+}
+
+// Inclusive scan over a wave (all lanes active): shifts by 1, 2, 4 and 8
+// within rows of 16 lanes, then the rows' totals. Six VALU steps, where a
+// shuffle goes through the LDS for each.
+template <typename T>
+__device__ __forceinline__ T wave_incl_scan(T x) {
+  x += dpp_or0<0x111, 0xf>(x);   // row_shr:1
+  x += dpp_or0<0x112, 0xf>(x);
+  x += dpp_or0<0x114, 0xf>(x);
+  x += dpp_or0<0x118, 0xf>(x);
+  x += dpp_or0<0x142, 0xa>(x);   // row_bcast:15 into rows 1 and 3
+  x += dpp_or0<0x143, 0xc>(x);   // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
 __device__ __forceinline__ float clampf(float x, float lo, float hi) {
   return fminf(fmaxf(x, lo), hi);
 }

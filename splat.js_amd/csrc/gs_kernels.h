@@ -69,7 +69,7 @@ struct BinArgs {
   uint64_t* totalKeys;    // device: keys before the budget
   uint2* ranges;          // numTiles
   uint32_t* tileOrder;    // numTiles: raster launch order, most keys first
-  double* stats;          // [3] += dropped keys
+  double* stats;          // [kStatDropped] += dropped keys
   SortScratch scratch;
 };
 
@@ -99,7 +99,7 @@ struct SegJob {
   uint32_t* numKeys;
   uint32_t* numVisible;
   uint64_t* totalKeys;
-  double* stats;          // [3] += dropped keys (atomically: views run together)
+  double* stats;          // [kStatDropped] += dropped keys (atomically: views run together)
   uint64_t* keys;         // cap: the scattered keys
   uint64_t* tmp;          // cap: merge scratch of segments over 1024 keys
   uint32_t* ids;          // cap: the raster values in sorted order
@@ -141,6 +141,19 @@ struct BinOut {
   int keyBytes;           // 8 (tile << 32 | depth), 4 (tile), 0 (none)
 };
 
+// A pass's statistics: kStatLines lines of 128 bytes, each with a part of
+// [0] sum |err|^2, [1] loss, [2] valid pixels, then one double of dropped
+// keys. A block adds its sums to the line of its index: atomics on one line
+// go through one after another, about 18 ns each, and a view of 2170 tiles
+// spent a quarter of its forward pass on them (979x546, 250k Gaussians: 61.1
+// -> 46.8 us).
+constexpr int kStatLines = 64, kStatLine = 16;
+constexpr int kStatDropped = kStatLines * kStatLine;
+constexpr int kStatDoubles = kStatDropped + 1;
+__device__ __forceinline__ double* stat_line(double* stats, uint32_t block) {
+  return stats + (block % kStatLines) * kStatLine;
+}
+
 struct RasterBufs {
   int recFmt;             // record colours: 0 f32 (64 B records), 1 bf16, 2 fp16 (48 B)
   const uint2* ranges;
@@ -154,7 +167,7 @@ struct RasterBufs {
   uint64_t* took;         // per 64-key chunk of a tile and wave: the keys that a lane of the wave took
                           // (training: written by the forward, read by the backward)
   const uint32_t* tgt;    // packed RGBA8 targets (all views)
-  double* stats;          // [0] sum |err|^2, [1] loss, [2] valid pixels
+  double* stats;          // kStatDoubles, or null
 };
 
 // a RasterBufs read from device memory, every pointer loaded by gs_global

@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kLossThreads) void k_ssim_fwd(Cam cam, SsimWin win,
   if (tid < 3) {
     double v = 0.0;
     for (int k = 0; k < kLossThreads / 64; k++) v += sStat[tid][k];
-    if (v != 0.0) atomicAdd(&b.stats[tid], v);
+    if (v != 0.0) atomicAdd(&stat_line(b.stats, blockIdx.x)[tid], v);
   }
 }
 

@@ -376,7 +376,7 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
     if (tid < 3) {
       double v = sStat[tid][0];
       for (int w = 1; w < S::kWaves; w++) v += sStat[tid][w];
-      if (v != 0.0) atomicAdd(&b.stats[tid], v);
+      if (v != 0.0) atomicAdd(&stat_line(b.stats, (uint32_t)tile)[tid], v);
     }
   }
 }

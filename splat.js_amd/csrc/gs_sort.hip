@@ -55,30 +55,6 @@ __device__ __forceinline__ uint64_t match_digit8(uint32_t d, uint64_t active) {
   return m;
 }
 
-// x of the lane a DPP control selects, 0 where it selects none
-template <int kCtrl, int kRows>
-__device__ __forceinline__ uint32_t dpp_or0(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, kRows, 0xf, false);
-}
-template <int kCtrl, int kRows>
-__device__ __forceinline__ uint64_t dpp_or0(uint64_t x) {
-  return ((uint64_t)dpp_or0<kCtrl, kRows>((uint32_t)(x >> 32)) << 32) | dpp_or0<kCtrl, kRows>((uint32_t)x);
-}
-
-// Inclusive scan over a wave (all lanes active): shifts by 1, 2, 4 and 8
-// within rows of 16 lanes, then the rows' totals. Six VALU steps, where a
-// shuffle goes through the LDS for each.
-template <typename T>
-__device__ __forceinline__ T wave_incl_scan(T x) {
-  x += dpp_or0<0x111, 0xf>(x);   // row_shr:1
-  x += dpp_or0<0x112, 0xf>(x);
-  x += dpp_or0<0x114, 0xf>(x);
-  x += dpp_or0<0x118, 0xf>(x);
-  x += dpp_or0<0x142, 0xa>(x);   // row_bcast:15 into rows 1 and 3
-  x += dpp_or0<0x143, 0xc>(x);   // row_bcast:31 into rows 2 and 3
-  return x;
-}
-
 constexpr int kItems = 8;
 constexpr int kRound = kBlock * kItems;   // keys per block round
 
@@ -371,7 +347,7 @@ __global__ __launch_bounds__(1024) void k_count_top(uint64_t* __restrict__ parti
     const uint64_t total = pre + x;
     *totalKeys = total;
     *numKeys = (uint32_t)(total < cap ? total : cap);
-    if (total > cap) stats[3] += (double)(total - cap);
+    if (total > cap) stats[kStatDropped] += (double)(total - cap);
   }
 }
 
@@ -987,7 +963,7 @@ __global__ __launch_bounds__(kScanThreads) void k_seg_scan(SegJob arg, const Seg
 #pragma unroll
     for (int k = 0; k < kWaves; k++) { r += wsB[k]; d += wsC[k].x; v += wsC[k].y; }
     *j.totalKeys = r;
-    if (d) atomicAdd(&j.stats[3], (double)d);   // the views' scans run together
+    if (d) atomicAdd(&j.stats[kStatDropped], (double)d);   // the views' scans run together
     *j.numVisible = v;
   }
   __syncthreads();

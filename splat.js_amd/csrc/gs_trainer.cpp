@@ -119,8 +119,8 @@ struct gs_trainer {
   float* ssimScratch = nullptr;  // 9 x maxPix SSIM partials (L1 + D-SSIM loss only)
   uint32_t* targets = nullptr;
   int64_t totalPx = 0;
-  double* stats = nullptr;      // training stats [4]
-  double* evalStats = nullptr;  // eval/view stats [4]
+  double* stats = nullptr;      // training stats (kStatDoubles)
+  double* evalStats = nullptr;  // eval/view stats (kStatDoubles)
   uint32_t* camGrad = nullptr;  // (numCams + 1) x 8 i32 camera gradient rows (trainer.js:173)
 
   std::vector<CamMeta> cams;
@@ -185,7 +185,7 @@ struct gs_pending {
   enum Kind { kLoss, kPsnr, kGaussians } kind = kLoss;
   int device = 0;
   hipEvent_t ev = nullptr;
-  double* stats = nullptr;     // pinned [4] (loss, psnr)
+  double* stats = nullptr;     // pinned kStatDoubles (loss, psnr)
   int64_t px = 0;              // pixels the loss window saw (loss)
   void* hP = nullptr;          // pinned parameter planes (gaussians)
   void* hSH = nullptr;         // pinned SH planes (gaussians)
@@ -213,6 +213,23 @@ int hipfail(gs_trainer* h, const char* what, hipError_t e) {
     hipError_t e_ = (expr);                           \
     if (e_ != hipSuccess) return hipfail(h, #expr, e_); \
   } while (0)
+
+// a statistics buffer's sums: sum |err|^2, loss, valid pixels, dropped keys
+void stat_sums(const double* raw, double (&s)[4]) {
+  for (int k = 0; k < 3; k++) s[k] = 0.0;
+  for (int l = 0; l < kStatLines; l++)
+    for (int k = 0; k < 3; k++) s[k] += raw[l * kStatLine + k];
+  s[3] = raw[kStatDropped];
+}
+
+hipError_t read_stats(const double* dev, double* out) {
+  double raw[kStatDoubles], s[4];
+  const hipError_t e = hipMemcpy(raw, dev, sizeof raw, hipMemcpyDeviceToHost);
+  if (e != hipSuccess) return e;
+  stat_sums(raw, s);
+  memcpy(out, s, sizeof s);
+  return e;
+}
 
 template <typename T>
 int dalloc(gs_trainer* h, T** p, size_t bytes) {
@@ -588,21 +605,22 @@ int eval_pass(gs_trainer* h, int ci, const double* R, const double* t, double g,
   m.b = b;
   refresh_cam(m);
   const Cam cam = make_cam_meta(h, m, h->shDeg);   // _camUniform: full SH degree (trainer.js:369)
-  HIPCK(hipMemsetAsync(h->evalStats, 0, 32, h->st));
+  HIPCK(hipMemsetAsync(h->evalStats, 0, 8 * kStatDoubles, h->st));
   int rc = run_raster(h, cam, 1, h->evalStats, true);   // forward, loss and backward
   if (rc) return rc;
   launch_cam_exposure(h->st, cam, h->img, h->targets, h->camGrad + 8 * ci);
   launch_cam_pose(h->st, h->o.gradAccum, true, cam, cam_pose_bufs(h, ci));
   HIPCK(hipGetLastError());
-  double s[4];
+  double raw[kStatDoubles], s[4];
   int32_t row[8];
   const size_t rows = h->cams.size() + 1;
-  HIPCK(hipMemcpyAsync(s, h->evalStats, 32, hipMemcpyDeviceToHost, h->st));
+  HIPCK(hipMemcpyAsync(raw, h->evalStats, sizeof raw, hipMemcpyDeviceToHost, h->st));
   HIPCK(hipMemcpyAsync(row, h->camGrad + 8 * ci, 32, hipMemcpyDeviceToHost, h->st));
   HIPCK(hipMemsetAsync(h->camGrad, 0, rows * 32, h->st));
-  HIPCK(hipMemsetAsync(h->stats, 0, 24, h->st));   // the loss window; the budget drops keep counting
+  HIPCK(hipMemsetAsync(h->stats, 0, 8 * kStatDropped, h->st));   // the loss window; the budget drops keep counting
   HIPCK(hipStreamSynchronize(h->st));
   h->pixelsSeen = 0;
+  stat_sums(raw, s);
   if (grad8) memcpy(grad8, row, sizeof row);
   if (psnr) {
     const double mse = s[0] / (std::max(1.0, s[2]) * 3.0);
@@ -780,7 +798,7 @@ int step_impl(gs_trainer* h, int ci, gs_debug_out* dbg) {
       (void)hipFree(dGF);
       (void)hipFree(dSG);
     }
-    if (dbg->stats) HIPCK(hipMemcpy(dbg->stats, h->stats, 32, hipMemcpyDeviceToHost));
+    if (dbg->stats) HIPCK(read_stats(h->stats, dbg->stats));
   }
   // trainer.js:468-470: one camera Adam step every 25 iterations after 1500
   if (h->o.camOpt && h->iter > 1500 && h->iter % 25 == 0) return apply_cam_grads(h);
@@ -1108,7 +1126,7 @@ int step_views_impl(gs_trainer* h, const int32_t* cams, int count, gs_debug_out*
     if (dGF && dbg[0].gradF) HIPCK(hipMemcpy(dbg[0].gradF, dGF, 64 * h->n, hipMemcpyDeviceToHost));
     if (dSG && dbg[0].shGrad && h->shC)
       HIPCK(hipMemcpy(dbg[0].shGrad, dSG, 4ull * h->shC * h->n, hipMemcpyDeviceToHost));
-    if (dbg[0].stats) HIPCK(hipMemcpy(dbg[0].stats, h->stats, 32, hipMemcpyDeviceToHost));
+    if (dbg[0].stats) HIPCK(read_stats(h->stats, dbg[0].stats));
   }
   if (dGF) (void)hipFree(dGF);
   if (dSG) (void)hipFree(dSG);
@@ -1378,8 +1396,8 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
   rc |= dalloc(h, &h->took, tookBytes);
   if (h->o.loss == GS_LOSS_L1_DSSIM) rc |= dalloc(h, &h->ssimScratch, (size_t)h->maxPix * 36);
   rc |= dalloc(h, &h->targets, tgt.size() * 4);
-  rc |= dalloc(h, &h->stats, 32);
-  rc |= dalloc(h, &h->evalStats, 32);
+  rc |= dalloc(h, &h->stats, 8 * kStatDoubles);
+  rc |= dalloc(h, &h->evalStats, 8 * kStatDoubles);
   rc |= dalloc(h, &h->camGrad, (size_t)(ncams + 1) * 32);
   // batched views: slot 0 is the single-view set, slots 1.. their own copies
   h->vslots.assign((size_t)h->o.viewsPerStep, gs_trainer::ViewSlot{});
@@ -1474,8 +1492,8 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
   HIPCK(hipMemset(h->SHM, 0, smb));
   HIPCK(hipMemset(h->SHV, 0, smb));
   HIPCK(hipMemset(h->accum, 0, (size_t)cap * 48));
-  HIPCK(hipMemset(h->stats, 0, 32));
-  HIPCK(hipMemset(h->evalStats, 0, 32));
+  HIPCK(hipMemset(h->stats, 0, 8 * kStatDoubles));
+  HIPCK(hipMemset(h->evalStats, 0, 8 * kStatDoubles));
   HIPCK(hipMemset(h->camGrad, 0, (size_t)(ncams + 1) * 32));
   for (size_t k = 1; k < h->vslots.size(); k++) HIPCK(hipMemset(h->vslots[k].accum, 0, (size_t)cap * 48));
   const uint32_t n32 = (uint32_t)n;
@@ -1614,16 +1632,16 @@ int gs_autotune(gs_trainer_t* h, const int32_t* cams, int32_t count, int32_t rep
     gs_tune_entry& en = out[i];
     set_shape(h, RasterShape{en.tile, en.batch});
     // warm-up pass: also gives the pass's keys and budget drops
-    if (hipMemsetAsync(h->evalStats, 0, 32, h->st) != hipSuccess) { rc = hipfail(h, "autotune", hipGetLastError()); break; }
+    if (hipMemsetAsync(h->evalStats, 0, 8 * kStatDoubles, h->st) != hipSuccess) { rc = hipfail(h, "autotune", hipGetLastError()); break; }
     rc = tune_pass(h, ci, count, activeDeg);
     if (rc) break;
-    double st4[4];
+    double drops = 0.0;
     uint32_t nk[kMaxViews] = {};
-    HIPCK(hipMemcpyAsync(st4, h->evalStats, 32, hipMemcpyDeviceToHost, h->st));
+    HIPCK(hipMemcpyAsync(&drops, h->evalStats + kStatDropped, 8, hipMemcpyDeviceToHost, h->st));
     if (count == 1) HIPCK(hipMemcpyAsync(nk, h->numKeys, 4, hipMemcpyDeviceToHost, h->st));
     else HIPCK(hipMemcpyAsync(nk, h->viewStats, 4ull * count, hipMemcpyDeviceToHost, h->st));
     HIPCK(hipStreamSynchronize(h->st));
-    en.dropped = (int64_t)st4[3];
+    en.dropped = (int64_t)drops;
     for (int k = 0; k < count; k++) en.keys += nk[k];
     HIPCK(hipEventRecord(e0, h->st));
     for (int r = 0; r < reps && rc == GS_OK; r++) rc = tune_pass(h, ci, count, activeDeg);
@@ -1640,7 +1658,7 @@ int gs_autotune(gs_trainer_t* h, const int32_t* cams, int32_t count, int32_t rep
   // the gradient sums of the passes and their statistics are discarded
   launch_fill_u32(h->st, (uint32_t*)h->accum, 12 * h->cap, 0u);
   for (const gs_trainer::ViewSlot& sl : h->vslots) launch_fill_u32(h->st, (uint32_t*)sl.accum, 12 * h->cap, 0u);
-  launch_fill_u32(h->st, (uint32_t*)h->evalStats, 8, 0u);
+  launch_fill_u32(h->st, (uint32_t*)h->evalStats, 2 * kStatDoubles, 0u);
   HIPCK(hipStreamSynchronize(h->st));
   if (rc) {
     set_shape(h, start);
@@ -1794,7 +1812,7 @@ static int pending_new(gs_trainer* h, gs_pending::Kind kind, gs_pending** out) {
   p->kind = kind;
   p->device = h->o.device;
   hipError_t e = hipEventCreateWithFlags(&p->ev, hipEventDisableTiming);
-  if (e == hipSuccess && kind != gs_pending::kGaussians) e = hipHostMalloc((void**)&p->stats, 32, hipHostMallocDefault);
+  if (e == hipSuccess && kind != gs_pending::kGaussians) e = hipHostMalloc((void**)&p->stats, 8 * kStatDoubles, hipHostMallocDefault);
   if (e != hipSuccess) {
     gs_pending_free(p);
     return hipfail(h, "readback setup", e);
@@ -1811,10 +1829,10 @@ int gs_read_loss_async(gs_trainer_t* h, gs_pending_t** out) {
   gs_pending* p = nullptr;
   int rc = pending_new(h, gs_pending::kLoss, &p);
   if (rc != GS_OK) return rc;
-  // copy the window's stats, then reset the window; stats[3] (the budget
-  // drops) keeps counting across windows (trainer.js:621-627)
-  hipError_t e = hipMemcpyAsync(p->stats, h->stats, 32, hipMemcpyDeviceToHost, h->st);
-  if (e == hipSuccess) e = hipMemsetAsync(h->stats, 0, 24, h->st);
+  // copy the window's stats, then reset the window; the budget drops behind
+  // it keep counting across windows (trainer.js:621-627)
+  hipError_t e = hipMemcpyAsync(p->stats, h->stats, 8 * kStatDoubles, hipMemcpyDeviceToHost, h->st);
+  if (e == hipSuccess) e = hipMemsetAsync(h->stats, 0, 8 * kStatDropped, h->st);
   if (e == hipSuccess) e = hipEventRecord(p->ev, h->st);
   if (e != hipSuccess) {
     gs_pending_free(p);
@@ -1835,17 +1853,17 @@ int gs_eval_cam_psnr_async(gs_trainer_t* h, int32_t ci, gs_pending_t** out) {
   const CamMeta& m = h->cams[ci];
   // the reference evaluates with the camera's training uniform (trainer.js:547)
   const Cam cam = make_cam_meta(h, m, m.activeDeg);
-  HIPCK(hipMemsetAsync(h->evalStats, 0, 32, h->st));
+  HIPCK(hipMemsetAsync(h->evalStats, 0, 8 * kStatDoubles, h->st));
   int rc = run_raster(h, cam, 1, h->evalStats);
   if (rc) return rc;
   gs_pending* p = nullptr;
   rc = pending_new(h, gs_pending::kPsnr, &p);
   if (rc != GS_OK) return rc;
-  hipError_t e = hipMemcpyAsync(p->stats, h->evalStats, 32, hipMemcpyDeviceToHost, h->st);
+  hipError_t e = hipMemcpyAsync(p->stats, h->evalStats, 8 * kStatDoubles, hipMemcpyDeviceToHost, h->st);
   // trainer.js:562, :570-571: the camera gradient rows are drained and the
   // training loss window is reset too
   if (e == hipSuccess) e = hipMemsetAsync(h->camGrad, 0, (h->cams.size() + 1) * 32, h->st);
-  if (e == hipSuccess) e = hipMemsetAsync(h->stats, 0, 24, h->st);
+  if (e == hipSuccess) e = hipMemsetAsync(h->stats, 0, 8 * kStatDropped, h->st);
   if (e == hipSuccess) e = hipEventRecord(p->ev, h->st);
   if (e != hipSuccess) {
     gs_pending_free(p);
@@ -1901,7 +1919,8 @@ int gs_pending_wait(gs_pending_t* p, gs_readback_result* out) {
     p->err = std::string("readback: ") + hipGetErrorString(e);
     return GS_E_HIP;
   }
-  const double* s = p->stats;
+  double s[4] = {};
+  if (p->stats) stat_sums(p->stats, s);
   switch (p->kind) {
     case gs_pending::kLoss:
       // trainer.js:621-630
@@ -2006,11 +2025,11 @@ int gs_read_step_stats(gs_trainer_t* h, gs_step_stats* out) {
   HIPCK(hipSetDevice(h->o.device));
   uint32_t nk = 0, nv = 0;
   uint32_t vs[2 * kMaxViews];
-  double s[4];
+  double drops = 0.0;
   HIPCK(hipMemcpyAsync(&nk, h->numKeys, 4, hipMemcpyDeviceToHost, h->st));
   HIPCK(hipMemcpyAsync(&nv, h->numVisible, 4, hipMemcpyDeviceToHost, h->st));
   if (h->lastViews > 0) HIPCK(hipMemcpyAsync(vs, h->viewStats, sizeof vs, hipMemcpyDeviceToHost, h->st));
-  HIPCK(hipMemcpyAsync(s, h->stats, 32, hipMemcpyDeviceToHost, h->st));
+  HIPCK(hipMemcpyAsync(&drops, h->stats + kStatDropped, 8, hipMemcpyDeviceToHost, h->st));
   HIPCK(hipStreamSynchronize(h->st));
   out->lastKeys = nk;
   out->lastVisible = nv;
@@ -2021,7 +2040,7 @@ int gs_read_step_stats(gs_trainer_t* h, gs_step_stats* out) {
       out->lastVisible += vs[kMaxViews + k];
     }
   }
-  out->overflowKeys = (int64_t)s[3];
+  out->overflowKeys = (int64_t)drops;
   return GS_OK;
 }
 
@@ -2058,9 +2077,9 @@ int gs_refine(gs_trainer_t* h, const gs_refine_opts* ro, gs_refine_result* out) 
     for (int t = 0; t < h->lastNumTiles; t++) out->maxTile = std::max<int64_t>(out->maxTile, rg[2 * t + 1] - rg[2 * t]);
   }
   {
-    double s[4];
-    HIPCK(hipMemcpy(s, h->stats, 32, hipMemcpyDeviceToHost));
-    out->overflow = (int64_t)s[3];
+    double drops = 0.0;
+    HIPCK(hipMemcpy(&drops, h->stats + kStatDropped, 8, hipMemcpyDeviceToHost));
+    out->overflow = (int64_t)drops;
   }
 
   // opacity logit and log-scales of every Gaussian (16 B each)
@@ -2342,7 +2361,7 @@ int gs_fd_grad64(gs_trainer_t* h, int32_t ci, const int64_t* gauss, const int32_
   CamMeta& meta = h->cams[ci];
   const int activeDeg = (int)std::min<int64_t>(h->shDeg, h->iter / 1000);
   const Cam cam = make_cam_meta(h, meta, activeDeg);
-  HIPCK(hipMemsetAsync(h->evalStats, 0, 32, h->st));
+  HIPCK(hipMemsetAsync(h->evalStats, 0, 8 * kStatDoubles, h->st));
   int rc = run_raster(h, cam, 1, h->evalStats);
   if (rc) return rc;
   // the samples' tile rectangles, one tile of margin each side
