@@ -35,12 +35,15 @@ struct SortScratch {
 // reference's scan covers 256 x 64 tiles, shaders.js:325); larger views use
 // the depth-then-tile radix sort.
 constexpr int kMaxSegTiles = 16384;
-// Gaussians per count/scatter block of the tile-segment strategy: at least
-// kSegMinGroup, so that the table has ceil(n / seg_group(n)) <=
-// min(kSegMaxRows, ceil(n / kSegMinGroup)) rows; from 256 * kSegMinGroup
-// Gaussians up, n / kSegBlocks, one 1024-thread block per CU of MI355X's 256
-constexpr int64_t kSegMinGroup = 2048;
-constexpr int64_t kSegMaxRows = 1024;
+// Gaussians per count/scatter block of the tile-segment strategy: n /
+// kSegBlocks, one 1024-thread block per CU of MI355X's 256, and at least
+// kSegMinGroup (a chunk below): a small view's passes last as long as one
+// block's keys, so it is split as far as the chunks go. Count and scatter at
+// groups of 2048, 1024, 512 and 256: 20k Gaussians at 320x240 8.3 + 13.4, 6.3
+// + 8.8, 5.6 + 6.8 and 5.4 + 6.2 us, 123k at 737x411 9.3 + 14.2, 7.7 + 11.3,
+// 6.2 + 9.5 and 6.2 + 8.1. A table has at most kSegBlocks rows, and no more
+// than ceil(n / kSegMinGroup) (seg_rows).
+constexpr int64_t kSegMinGroup = 256;
 constexpr int64_t kSegBlocks = 256;
 // Gaussians per chunk of the block balancing: count/scatter blocks take whole
 // chunks, as many as give each block an equal share of the work (keys plus
@@ -48,6 +51,11 @@ constexpr int64_t kSegBlocks = 256;
 constexpr int64_t kSegChunk = 256;
 int64_t seg_group(int64_t n);
 int seg_blocks(int64_t n);   // count/scatter blocks of the tile-segment binning
+// table rows that hold seg_blocks(n) for every n <= cap
+constexpr int64_t seg_rows(int64_t cap) {
+  const int64_t r = (cap + kSegMinGroup - 1) / kSegMinGroup;
+  return r < kSegBlocks ? r : kSegBlocks;
+}
 
 struct BinArgs {
   int mode;               // 0 depth-then-tile, 1 global64, 2 tile segments

@@ -791,41 +791,28 @@ __global__ __launch_bounds__(kBlock) void k_seg_colscan(SegJob arg, const SegJob
   const int t = blockIdx.x * 16 + tl;
   const int per = (nb + 15) / 16;
   const int b0 = q * per, b1 = b0 + per < nb ? b0 + per : nb;
-  // up to kRegRows rows per thread (tables of up to 256 rows: 1M Gaussians)
-  // stay in registers: one batch of independent loads, no second read
-  constexpr int kRegRows = 16;
+  // a thread's rows stay in registers: one batch of independent loads
+  constexpr int kRegRows = (int)(kSegBlocks / 16);
+  static_assert(kSegBlocks % 16 == 0, "sixteenths of the rows");
   uint32_t v[kRegRows];
   uint32_t sum = 0;
-  if (per <= kRegRows) {
 #pragma unroll
-    for (int k = 0; k < kRegRows; k++) {
-      const int b = b0 + k;
-      v[k] = (t < numTiles && b < b1) ? table[(int64_t)b * numTiles + t] : 0u;
-      sum += v[k];
-    }
-  } else if (t < numTiles) {
-    for (int b = b0; b < b1; b++) sum += table[(int64_t)b * numTiles + t];
+  for (int k = 0; k < kRegRows; k++) {
+    const int b = b0 + k;
+    v[k] = (t < numTiles && b < b1) ? table[(int64_t)b * numTiles + t] : 0u;
+    sum += v[k];
   }
   part[q][tl] = sum;
   __syncthreads();
   if (t >= numTiles) return;
   uint32_t run = 0;
   for (int k = 0; k < q; k++) run += part[k][tl];
-  if (per <= kRegRows) {
 #pragma unroll
-    for (int k = 0; k < kRegRows; k++) {
-      const int b = b0 + k;
-      if (b < b1) {
-        table[(int64_t)b * numTiles + t] = run;
-        run += v[k];
-      }
-    }
-  } else {
-    for (int b = b0; b < b1; b++) {
-      uint32_t* p = table + (int64_t)b * numTiles + t;
-      const uint32_t x = *p;
-      *p = run;
-      run += x;
+  for (int k = 0; k < kRegRows; k++) {
+    const int b = b0 + k;
+    if (b < b1) {
+      table[(int64_t)b * numTiles + t] = run;
+      run += v[k];
     }
   }
   if (q == 15) tileCnt[t] = run;
@@ -882,7 +869,7 @@ __global__ __launch_bounds__(kScanThreads) void k_seg_scan(SegJob arg, const Seg
   uint32_t c[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; k++) c[k] = t0 + k < numTiles ? tileCnt[t0 + k] : 0u;
-  const uint32_t vis = tid < nb ? j.visPart[tid] : 0u;   // nb <= kSegMaxRows = kScanThreads
+  const uint32_t vis = tid < nb ? j.visPart[tid] : 0u;   // nb <= kSegBlocks
   // the count pass has read the chunk key sums: clear them for the next
   // projection to fill
   const int64_t nChunks = (j.n + kSegChunk - 1) / kSegChunk;
@@ -1440,11 +1427,8 @@ static void radix_sort(hipStream_t st, const SortScratch& s, const KeyT* kin, co
 }
 
 int64_t seg_group(int64_t n) {
-  // Gaussians per count/scatter block: n / kSegBlocks (one block per CU),
-  // at least kSegMinGroup; the blocks take whole chunks by cost, so the
-  // group only sets their number. kSegBlocks <= kSegMaxRows keeps the table
-  // within its rows.
-  static_assert(kSegBlocks <= kSegMaxRows, "block count above the table's rows");
+  // the blocks take whole chunks by cost, so the group only sets their number
+  static_assert(kSegBlocks <= kScanThreads, "one scan thread per block");
   const int64_t g = (n + kSegBlocks - 1) / kSegBlocks;
   return g > kSegMinGroup ? g : kSegMinGroup;
 }

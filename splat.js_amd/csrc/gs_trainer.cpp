@@ -1370,8 +1370,7 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
   rc |= dalloc(h, &h->sort.nDepth, 4);
   rc |= dalloc(h, &h->sort.tileCnt, (size_t)h->maxTiles * 4);
   if (h->o.sortMode == GS_SORT_TILE_SEGMENTS) {
-    // rows = ceil(n / seg_group(n)) <= min(kSegMaxRows, ceil(cap / kSegMinGroup)) for every n <= cap
-    const int64_t rows = std::min<int64_t>(kSegMaxRows, (cap + kSegMinGroup - 1) / kSegMinGroup);
+    const int64_t rows = seg_rows(cap);
     // (the segment path takes views of at most kMaxSegTiles tiles)
     rc |= dalloc(h, &h->sort.segTable, (size_t)rows * std::min(h->maxTiles, kMaxSegTiles) * 4);
     rc |= dalloc(h, &h->sort.visPart, (size_t)rows * 4);
@@ -1428,7 +1427,7 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
   // copies would pass kBatchedBinBytes (then the views bin one after
   // another through the shared buffers).
   if (rc == 0 && h->o.viewsPerStep > 1 && h->o.sortMode == GS_SORT_TILE_SEGMENTS) {
-    const int64_t rows = std::min<int64_t>(kSegMaxRows, (cap + kSegMinGroup - 1) / kSegMinGroup);
+    const int64_t rows = seg_rows(cap);
     const size_t segTiles = (size_t)std::min(h->maxTiles, kMaxSegTiles);
     const size_t chunkBytes = (size_t)((cap + kSegChunk - 1) / kSegChunk) * 4;
     const size_t per = (size_t)cap * 12 + chunkBytes + (size_t)(2 * rows + 1) * 4 + (size_t)rows * segTiles * 4 +
