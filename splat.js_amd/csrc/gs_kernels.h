@@ -322,6 +322,12 @@ struct RefineOp {
 };
 
 // q[i] = (opacity logit, log-scale x, y, z) for i < n
+// Rows [first, first + count) of the parameters (16 floats each) and of the SH
+// coefficients (C floats each; fmt 0 f32 planes, 1 bf16, 2 fp16) into out.
+void launch_param_rows(hipStream_t st, int64_t cap, int64_t first, int64_t count, const float4* P, float* out);
+void launch_sh_rows(hipStream_t st, int fmt, int64_t cap, int64_t first, int64_t count, int C, const void* SH,
+                    float* out);
+
 void launch_refine_gather(hipStream_t st, int64_t n, int64_t cap, const float4* P, float4* q);
 void launch_refine_apply(hipStream_t st, int deg, int prec, int64_t cap, const RefineOp* ops, int64_t count,
                          float4* P, void* M, void* V, void* SH, void* SHM, void* SHV);

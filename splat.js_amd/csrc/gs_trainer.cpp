@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/splat_gs.h"
+#include "gs_hostcopy.h"
 #include "gs_kernels.h"
 
 using namespace gs;
@@ -93,6 +94,9 @@ struct gs_trainer {
   int maxTiles = 0;      // tiles of the largest view at the smallest tile size (8): every shape fits
   int64_t maxPix = 0;
   RasterShape shape{kDefaultTile, kDefaultBatch};   // raster tile side and LDS batch
+
+  HostRing ring;                        // pinned blocks of the large synchronous reads
+  std::shared_ptr<StatPool> statPool;   // pinned blocks of the loss and PSNR reads
 
   std::vector<void*> allocs;
   float4* P = nullptr;
@@ -179,13 +183,15 @@ struct gs_trainer {
 };
 
 // One asynchronous readback: pinned host copies, filled on the trainer's
-// stream, and an event behind them. It owns everything it touches, so it
+// stream, and an event behind them. It owns everything it touches (its
+// statistics block comes from a pool that it shares with the trainer), so it
 // outlives its trainer and its wait can run on any thread.
 struct gs_pending {
   enum Kind { kLoss, kPsnr, kGaussians } kind = kLoss;
   int device = 0;
   hipEvent_t ev = nullptr;
   double* stats = nullptr;     // pinned kStatDoubles (loss, psnr)
+  std::shared_ptr<StatPool> pool;   // where stats and ev go back to (loss, psnr)
   int64_t px = 0;              // pixels the loss window saw (loss)
   void* hP = nullptr;          // pinned parameter planes (gaussians)
   void* hSH = nullptr;         // pinned SH planes (gaussians)
@@ -1259,6 +1265,7 @@ void gs_destroy(gs_trainer_t* h) {
   if (h->evJoin) (void)hipEventDestroy(h->evJoin);
   for (hipEvent_t e : h->evBin)
     if (e) (void)hipEventDestroy(e);
+  h->ring.release();
   if (h->st) (void)hipStreamDestroy(h->st);
   delete h;
 }
@@ -1720,11 +1727,19 @@ int gs_render(gs_trainer_t* h, const gs_camera* c, int32_t trainMode, int64_t of
   if (c->w <= 0 || c->h <= 0) return fail(h, GS_E_ARG, "renderView: empty view");
   if (trainMode && (offset < 0 || offset + (int64_t)c->w * c->h > h->totalPx))
     return fail(h, GS_E_ARG, "renderView: target offset outside the packed targets");
+  HIPCK(hipSetDevice(h->o.device));
   const Cam cam = make_cam(h, *c, trainMode, offset, h->shDeg);
   int rc = run_raster(h, cam, trainMode ? 1 : 0, h->evalStats);
   if (rc) return rc;
-  HIPCK(hipMemcpyAsync(rgba, h->img, 16ull * c->w * c->h, hipMemcpyDeviceToHost, h->st));
-  HIPCK(hipStreamSynchronize(h->st));
+  const size_t bytes = 16ull * c->w * c->h, block = HostRing::kSlotBytes;
+  const auto size = [&](int k) { return std::min(block, bytes - k * block); };
+  const hipError_t e = ring_copy(
+      h->ring, h->st, (int)((bytes + block - 1) / block), std::min(bytes, block),
+      [&](int k, char* slot) {
+        return hipMemcpyAsync(slot, (const char*)h->img + k * block, size(k), hipMemcpyDeviceToHost, h->st);
+      },
+      [&](int k, const char* slot) { memcpy((char*)rgba + k * block, slot, size(k)); });
+  if (e != hipSuccess) return hipfail(h, "renderView", e);
   return GS_OK;
 }
 
@@ -1799,9 +1814,31 @@ int gs_read_cam_grads(gs_trainer_t* h, int32_t* out, int32_t count) {
 
 int gs_read_gaussians(gs_trainer_t* h, float* params, float* sh) {
   if (!h) return GS_E_ARG;
-  gs_pending* p = nullptr;
-  gs_readback_result r{};
-  return wait_pending(h, gs_read_gaussians_async(h, params, sh, &p), p, &r);
+  if (!h->ready) return fail(h, GS_E_ARG, "setup() has not been called");
+  HIPCK(hipSetDevice(h->o.device));
+  // whole rows to a block: kP blocks of parameters, then kS of coefficients
+  const int64_t n = h->n, C = sh ? h->shC : 0;
+  const int64_t rowsP = (int64_t)(HostRing::kSlotBytes / 64), rowsS = C ? (int64_t)(HostRing::kSlotBytes / (4 * C)) : 1;
+  const int kP = params ? (int)((n + rowsP - 1) / rowsP) : 0, kS = C ? (int)((n + rowsS - 1) / rowsS) : 0;
+  const size_t most = 4 * (size_t)std::max(kP ? 16 * std::min(rowsP, n) : 0, kS ? C * std::min(rowsS, n) : 0);
+  const hipError_t e = ring_copy(
+      h->ring, h->st, kP + kS, most,
+      [&](int k, char* slot) {
+        if (k < kP) {
+          launch_param_rows(h->st, h->cap, k * rowsP, std::min(rowsP, n - k * rowsP), h->P, (float*)slot);
+        } else {
+          const int64_t first = (k - kP) * rowsS;
+          launch_sh_rows(h->st, h->shFmt, h->cap, first, std::min(rowsS, n - first), (int)C, h->SH, (float*)slot);
+        }
+        return hipGetLastError();
+      },
+      [&](int k, const char* slot) {
+        const bool p = k < kP;
+        const int64_t rows = p ? rowsP : rowsS, width = p ? 16 : C, first = (p ? k : k - kP) * rows;
+        memcpy((p ? params : sh) + first * width, slot, (size_t)(4 * width * std::min(rows, n - first)));
+      });
+  if (e != hipSuccess) return hipfail(h, "readGaussians", e);
+  return GS_OK;
 }
 
 // ---- asynchronous readbacks ----
@@ -1810,8 +1847,17 @@ static int pending_new(gs_trainer* h, gs_pending::Kind kind, gs_pending** out) {
   gs_pending* p = new gs_pending();
   p->kind = kind;
   p->device = h->o.device;
-  hipError_t e = hipEventCreateWithFlags(&p->ev, hipEventDisableTiming);
-  if (e == hipSuccess && kind != gs_pending::kGaussians) e = hipHostMalloc((void**)&p->stats, 8 * kStatDoubles, hipHostMallocDefault);
+  hipError_t e = hipSuccess;
+  if (kind == gs_pending::kGaussians) {
+    e = hipEventCreateWithFlags(&p->ev, hipEventDisableTiming);
+  } else {
+    if (!h->statPool) h->statPool = std::make_shared<StatPool>(h->o.device, 8 * kStatDoubles);
+    p->pool = h->statPool;
+    StatPool::Block b;
+    e = p->pool->get(b);
+    p->stats = b.stats;
+    p->ev = b.ev;
+  }
   if (e != hipSuccess) {
     gs_pending_free(p);
     return hipfail(h, "readback setup", e);
@@ -1966,11 +2012,13 @@ const char* gs_pending_error(gs_pending_t* p) { return p ? p->err.c_str() : "nul
 void gs_pending_free(gs_pending_t* p) {
   if (!p) return;
   (void)hipSetDevice(p->device);
-  if (p->ev) {
-    (void)hipEventSynchronize(p->ev);   // a copy in flight still targets the pinned buffers
+  if (p->ev) (void)hipEventSynchronize(p->ev);   // a copy in flight still targets the pinned buffers
+  if (p->pool) {
+    StatPool::Block b{p->stats, p->ev};
+    if (p->ev) p->pool->put(b);
+  } else if (p->ev) {
     (void)hipEventDestroy(p->ev);
   }
-  if (p->stats) (void)hipHostFree(p->stats);
   if (p->hP) (void)hipHostFree(p->hP);
   if (p->hSH) (void)hipHostFree(p->hSH);
   delete p;

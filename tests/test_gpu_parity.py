@@ -639,3 +639,55 @@ def test_gradient_terms_beyond_the_fixed_point_clamp(gain):
     # the camera struct holds the log gain in f32
     cams = [dict(c, g=float(np.float32(math.log(gain)))) for c in cams]
     _run_pair(params, sh, cams, images, W, H, radius, opts, 3, steps=2, start_iter=5000)
+
+
+@pytest.mark.parametrize("precision", [gsabi.GS_PREC_F32, gsabi.GS_PREC_BF16, gsabi.GS_PREC_FP16])
+@pytest.mark.parametrize("n,deg", [(1, 3), (32768, 0), (32769, 1), (11651, 3), (11650, 3), (600001, 2)])
+def test_gaussians_read_in_blocks(n, deg, precision):
+    """readGaussians hands 2 MB blocks of whole rows through a ring of 8: one
+    row, one whole block (32768 rows of parameters; 11650 of degree 3), one
+    row more, and several times around the ring. The rows are those set up
+    (coefficients as the storage format rounds them, which the asynchronous
+    read, a host loop over the planes, gives too)."""
+    print(n, deg, precision, flush=True)
+    rng = np.random.default_rng(n + deg)
+    K = scenes.sh_k(deg)
+    p = np.zeros((n, 16), np.float32)
+    p[:, :14] = rng.normal(0, 1, (n, 14))
+    sh = rng.normal(0, 1, (n, 3 * K)).astype(np.float32) if K else None
+    cams = [{"imgIdx": 0, "R": [1, 0, 0, 0, 1, 0, 0, 0, 1], "t": [0, 0, 0], "f": 16.0, "cx": 8, "cy": 8, "w": 16, "h": 16}]
+    images = [{"tw": 16, "th": 16, "rgb": np.full((256, 3), 0.5, np.float32)}]
+    t = _trainer(p, sh, cams, images, 16, 16, 1.0, {}, shDeg=deg, precision=precision, maxSplats=n + 77)
+    got, again, ref = t.readGaussians(), t.readGaussians(), t.read_gaussians_async().wait()
+    t.destroy()
+    for g in (got, again):
+        np.testing.assert_array_equal(g["data"].view(np.uint32), p.view(np.uint32))
+        if K:
+            np.testing.assert_array_equal(g["sh"].view(np.uint32), ref["sh"].view(np.uint32))
+            if precision == gsabi.GS_PREC_F32:
+                np.testing.assert_array_equal(g["sh"], sh)
+
+
+@pytest.mark.parametrize("W,H", [(1, 1), (512, 256), (257, 511), (1921, 1081)])
+def test_view_read_in_blocks(W, H):
+    """A rendered view comes in the same blocks: one pixel, one whole block,
+    one pixel short of it, and several times around the ring; the image is
+    the training forward's, which is read in one copy."""
+    rng = np.random.default_rng(W)
+    n, f = 500, float(W)
+    p = np.zeros((n, 16), np.float32)
+    z = rng.uniform(2.0, 4.0, n)
+    p[:, 0] = rng.uniform(-0.5, 0.5, n) * W / f * z
+    p[:, 1] = rng.uniform(-0.5, 0.5, n) * H / f * z
+    p[:, 2] = z
+    p[:, 3:6] = np.log(0.2)
+    p[:, 6] = 1.0
+    p[:, 10:14] = rng.normal(0, 1, (n, 4))
+    cams = [{"imgIdx": 0, "R": [1, 0, 0, 0, 1, 0, 0, 0, 1], "t": [0, 0, 0], "f": f, "cx": W / 2, "cy": H / 2, "w": W, "h": H}]
+    images = [{"tw": W, "th": H, "rgb": np.full((W * H, 3), 0.5, np.float32)}]
+    t = _trainer(p, None, cams, images, W, H, 1.0, {}, shDeg=0)
+    a, b = t.renderView(cams[0]), t.renderView(cams[0])
+    ref = t.step_debug(0, want=("img",))["img"]
+    t.destroy()
+    for v in (a, b):
+        np.testing.assert_array_equal(v.reshape(-1).view(np.uint32), ref.reshape(-1).view(np.uint32))
