@@ -172,7 +172,7 @@ struct RasterBufs {
   float* T;
   uint32_t* end;
   float4* gC;             // dL/dC, w = valid
-  uint64_t* took;         // per 64-key chunk of a tile and wave: the keys that a lane of the wave took
+  uint64_t* took;         // per 64-key chunk of a tile and 4x4 pixels: the keys that one of the pixels took
                           // (training: written by the forward, read by the backward)
   const uint32_t* tgt;    // packed RGBA8 targets (all views)
   double* stats;          // kStatDoubles, or null

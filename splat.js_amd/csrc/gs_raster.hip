@@ -27,12 +27,16 @@
 // its pixels down to the first key (each wave from the largest `end` of its
 // own pixels), recomputing each pixel's transmittance
 // in front of a splat from the stored final T (Tb = Ta/(1-a), through one
-// reciprocal that also scales the colour-behind sum S). A wave visits exactly
-// the keys that some lane of it took in the forward, which leaves one word per
-// 64 keys and wave for this (RasterBufs::took).
-// Per key, the 10 screen-space gradient terms of the wave's 64 pixels are
-// summed (DPP adds, then the wave's own LDS scratch; WaveRed below) and added
-// to the Gaussian's accumulator with one atomic per term per wave:
+// reciprocal that also scales the colour-behind sum S). The 16-lane groups of
+// a wave (4x4 pixels each) walk lists of their own: the keys that some lane
+// of the group took in the forward, which leaves one word per 64 keys and
+// group for this (RasterBufs::took). A wave is done with a batch of 128 keys
+// when its longest list is: a splat that misses a group costs it nothing,
+// where a walk of the whole wave's keys left half of the lanes idle.
+// Per visit, the 10 screen-space gradient terms of each group's 16 pixels are
+// summed (one DPP step, then the wave's own LDS scratch; WaveRed below) and
+// added to the batch's sums in LDS; these go to the Gaussians' accumulators
+// with one atomic per key, term and tile once the batch is done:
 //   GS_ACCUM_FIXED: each pixel's term is converted to i32 first,
 //                   i32(clamp(v * 16384, -1e9, 1e9)), exactly as the
 //                   reference's atomicAdd on atomic<i32> (shaders.js:529-541);
@@ -53,12 +57,15 @@
 // What bounds both visit loops is instruction issue: vector instructions
 // where the chip is full, and on small images, with about one wave per SIMD,
 // every instruction, scalar ones included (~4 cycles each there). So the
-// masks of a visit live in scalar registers, with one instruction to clear a
-// bit, and the records of a chunk lie in the order of the walk, which makes
-// it a find-first-bit both ways. Measured with the reduction through LDS and
-// the took words (1M Gaussians, 1600x900, ~3.25M keys): forward and backward
-// in one launch 626 -> 538 us; 8 views at once 4.32 -> 3.84 ms; the forward
-// alone at 1237x933, 2.0M keys, 155 -> 132 us, the backward 439 -> 382.
+// masks of a forward visit live in scalar registers, with one instruction to
+// clear a bit. Backward with lists per group against a walk of the wave's
+// keys with an atomic per wave: 20k Gaussians at 320x240 87 -> 64 us, 600k at
+// 1237x933 389 -> 315; forward and backward in one launch, 160 Gaussians at
+// 64x64 28 -> 24, 123k at 737x411 93 -> 79, 1M at 1600x900 566 -> 543, 8 views
+// of 1M 3865 -> 3745. Where splats cover whole tiles the lists of a wave are
+// all alike and their making is extra work: 1M large Gaussians, two views
+// at 1920x1080, 883 -> 985. Added to the Gaussians directly, the groups'
+// sums were bound by the rate of atomics (389 -> 787 at 1237x933).
 #include <type_traits>
 
 #include "gs_kernels.h"
@@ -69,7 +76,7 @@ __device__ __forceinline__ int tile_of_block(const RasterBufs& b) { return (int)
 
 // Shape of a raster launch: kT x kT pixel tiles, one thread per pixel, in
 // waves of 8x8 pixel blocks (wave w: block column w % (kT/8), block row
-// w / (kT/8); lane l is pixel (l & 7, l >> 3) of its block), and kB keys
+// w / (kT/8); each 16 lanes a 4x4 block of it, row by row), and kB keys
 // staged in LDS per round, in chunks of 64 keys (one ballot word each).
 // Each key carries 4 cover bits, one per quadrant of the tile (kT/2 x kT/2
 // pixels, bit 2 row + column): a wave tests its quadrant's bit (at kT = 16
@@ -83,11 +90,11 @@ struct Shape {
   static constexpr int kChunks = kB / 64;
   static constexpr int kBW = kT / 8;            // 8x8 blocks per tile row
   static constexpr int kMasks = kT == 8 ? 1 : 4;
-  // occupancy the persistent forward-and-backward launch is compiled for: 8
-  // waves per SIMD (at most 64 VGPRs; left free, the compiler takes up to 80
-  // there and the grid, sized by occupancy, shrinks); 8-pixel tiles with
-  // 128- or 256-key batches are held below that by their LDS anyway
-  static constexpr int kBwdWavesPerEU = (kT == 8 && kB > 64) ? 1 : 8;
+  // occupancy the launches with a backward are compiled for: 8 waves per SIMD
+  // (at most 64 VGPRs; left free, the compiler takes 72, and the persistent
+  // grid, sized by occupancy, shrinks); 8-pixel tiles are held below that by
+  // their LDS anyway
+  static constexpr int kBwdWavesPerEU = kT == 8 ? 1 : 8;
   static_assert((kT == 8 || kT == 16 || kT == 32) && (kB == 64 || kB == 128 || kB == 256), "raster shape");
   __device__ static int mask_slot(int w) {
     if constexpr (kT == 8) {
@@ -102,14 +109,20 @@ struct Shape {
 // LDS of the raster passes, carved from one array that the kernel declares,
 // so a launch that runs both passes holds the larger layout, not both.
 // Forward: records sA, sB, sC (16 B each per key), the chunk masks per
-// quadrant, the loss partials; backward: records sA-sD, the chunk masks per
-// wave, the block's largest end. Sizes in float4.
+// quadrant, the loss partials; backward: the records of a batch of 128 keys
+// and one that no lane takes, the waves' reduction scratch, the groups'
+// lists, the batch's gradient sums, the block's largest end. Sizes in float4.
+// 128 keys keep a block of 16-pixel tiles at 18.8 KB, eight to a CU.
 constexpr int kRedStride = 68;   // words between a wave's 64-word rows (see WaveRed)
+constexpr int kGroups = 4;       // 16-lane groups of a wave, each a 4x4 pixel block
 template <class S>
 struct RasterLds {
+  static constexpr int kKeys = S::B < 128 ? S::B : 128;   // keys per batch of the backward
   static constexpr int kFwd = 3 * S::B + (S::kChunks * S::kMasks * 8 + 3 * S::kWaves * 8 + 15) / 16;
   static constexpr int kRed = S::kWaves * 5 * kRedStride / 4;   // the waves' reduction scratch
-  static constexpr int kBwd = 3 * S::B + kRed + (S::kChunks * S::kWaves * 8 + 4 + 15) / 16;
+  static constexpr int kLists = S::kWaves * kGroups * kKeys / 16;   // a byte per key and group
+  static constexpr int kSums = (kKeys + 1) * 10 / 4 + 1;            // the batch's gradient sums
+  static constexpr int kBwd = 3 * (kKeys + 1) + kRed + kLists + kSums + 1;   // one record more: nobody's
   static constexpr int kBoth = kFwd > kBwd ? kFwd : kBwd;
 };
 
@@ -131,8 +144,8 @@ __device__ __forceinline__ PixelMap pixel_of_thread(const Cam& cam, int tile, in
   const int tx = tile % cam.tilesX, ty = tile / cam.tilesX;
   const int w = tid >> 6, l = tid & 63;
   PixelMap m;
-  m.x = tx * S::T + (w % S::kBW) * 8 + (l & 7);
-  m.y = ty * S::T + (w / S::kBW) * 8 + (l >> 3);
+  m.x = tx * S::T + (w % S::kBW) * 8 + (l & 3) + 4 * ((l >> 4) & 1);
+  m.y = ty * S::T + (w / S::kBW) * 8 + ((l >> 2) & 3) + 4 * (l >> 5);
   return m;
 }
 
@@ -159,11 +172,21 @@ __device__ __forceinline__ void clear_bit(uint64_t& m, int bit) {
   asm("s_bitset0_b64 %0, %1" : "+s"(m) : "s"(bit));
 }
 
-// the same when `mask` is empty (left to the compiler: five instructions)
-__device__ __forceinline__ void clear_bit_if_none(uint64_t& m, int bit, uint64_t mask) {
-  asm("s_cmp_lg_u64 %1, 0\n\ts_cbranch_scc1 .Lgs_some%=\n\ts_bitset0_b64 %0, %2\n.Lgs_some%=:"
-      : "+s"(m) : "s"(mask), "s"(bit) : "scc");
+// the OR over the first n lanes (the others hold 0), in a scalar register
+template <int n>
+__device__ __forceinline__ uint32_t or_lanes(uint32_t v) {
+  v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, false);   // row_ror 8, 4, 2, 1
+  v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xf, 0xf, false);
+  v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x122, 0xf, 0xf, false);
+  v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x121, 0xf, 0xf, false);
+  uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)v, 0);
+#pragma unroll
+  for (int l = 16; l < n; l += 16) r |= (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+  return r;
 }
+
+// `old` with lane `lane` set to v (both uniform)
+__device__ int write_lane(int v, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
@@ -215,14 +238,14 @@ __device__ __forceinline__ float4 record_colour(int recFmt, const float4& r1, fl
   return make_float4(dec16<1>(rg), dec16<1>(rg >> 16), dec16<1>(bl), w);
 }
 
-// First word (of one per wave) of RasterBufs::took for 64-key chunk `c`
+// First word (of one per 4x4 block, a wave's four next to each other) of RasterBufs::took for 64-key chunk `c`
 // (below the tile's keys / 64, rounded up) of the tile whose keys start at s.
 // Tiles lie in key order, so the rows of two
 // tiles never overlap: s / 64 grows by at least the earlier tile's chunks
 // less one, and the tile index by one.
 template <class S>
 __device__ __forceinline__ size_t took_word(uint32_t s, int tile, uint32_t c) {
-  return ((size_t)(s >> 6) + (uint32_t)tile + c) * S::kWaves;
+  return ((size_t)(s >> 6) + (uint32_t)tile + c) * (S::kWaves * kGroups);
 }
 
 // One tile of the forward pass, by the whole 256-thread block. The block's
@@ -282,7 +305,7 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
     if (run != 0ull) {
       for (int c = 0; c < S::kChunks; c++) {
         uint64_t m = uniform64(sMask[c][mslot]);
-        uint64_t took = m;   // kTook: keys of the chunk that some lane takes
+        int tkLo = 0, tkHi = 0;   // kTook: lane k holds the lanes that take key k of the chunk
         while (m) {
           const int bit = (int)__builtin_ctzll(m);
           clear_bit(m, bit);
@@ -299,11 +322,10 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
           // and the exp below needs its argument in [-87, 0]
           const float ee = clamp_e(fmaf(0.5f, t2, (a.w * dx) * dy));
           const uint64_t live = run & wave_ballot(ee <= cut.eCut);
-          uint64_t take = 0ull;
           if (live != 0ull) {
             const float araw = bb.y * gs_expf_raster(-ee);
             const float alpha = fminf(0.99f, araw);
-            take = live & wave_ballot(alpha >= cut.aMin);
+            const uint64_t take = live & wave_ballot(alpha >= cut.aMin);
             if (__builtin_amdgcn_inverse_ballot_w64(take)) {
               const float4 c4 = lds_at<float4>(sC + 64 * c, jo);
               const float w = T * alpha;
@@ -315,6 +337,10 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
             // T only falls here, so a lane reaches T < 1e-4 on this splat
             // exactly when it is still running and now below; that happens
             // once per pixel, so its bookkeeping sits behind a scalar branch
+            if (kTook) {
+              tkLo = write_lane((int)(uint32_t)take, bit, tkLo);
+              tkHi = write_lane((int)(uint32_t)(take >> 32), bit, tkHi);
+            }
             const uint64_t fin = run & wave_ballot(T < 1e-4f);
             if (fin != 0ull) {
               if (__builtin_amdgcn_inverse_ballot_w64(fin)) end = base + (uint32_t)(64 * c + bit) + 1u;
@@ -322,10 +348,16 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
               if (run == 0ull) m = 0ull;
             }
           }
-          if (kTook) clear_bit_if_none(took, bit, take);
         }
-        if (kTook && lane == 0 && 64u * (uint32_t)c < cnt)
-          b.took[took_word<S>(s, tile, ((base - s) >> 6) + (uint32_t)c) + wv] = took;
+        if (kTook && 64u * (uint32_t)c < cnt) {
+          const uint64_t w0 = wave_ballot(((uint32_t)tkLo & 0xffffu) != 0u), w1 = wave_ballot(((uint32_t)tkLo >> 16) != 0u);
+          const uint64_t w2 = wave_ballot(((uint32_t)tkHi & 0xffffu) != 0u), w3 = wave_ballot(((uint32_t)tkHi >> 16) != 0u);
+          if (lane == 0) {
+            ulonglong2* tw = (ulonglong2*)(b.took + took_word<S>(s, tile, ((base - s) >> 6) + (uint32_t)c) + wv * kGroups);
+            tw[0] = make_ulonglong2(w0, w1);
+            tw[1] = make_ulonglong2(w2, w3);
+          }
+        }
         if (run == 0ull) break;
       }
       if (__builtin_amdgcn_inverse_ballot_w64(run)) end = base + cnt;
@@ -381,8 +413,8 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
   }
 }
 
-// ---- wave reduction of a visit's 10 values ----
-// A visit's terms are summed over the wave's 64 lanes in two steps:
+// ---- reduction of a visit's 10 values over each 16-lane group ----
+// A visit's terms are summed over a group (a DPP row) in two steps:
 //  1. l ^ 15 (row_mirror, across bit 3 of the lane index) as two DPP adds per
 //     output, each writing one half of the row through the DPP bank mask (no
 //     selects): lanes 0-7 of each 16-lane row keep values 0-4, lanes 8-15
@@ -390,14 +422,13 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
 //  2. through the wave's own LDS scratch: register i goes to word 68 i +
 //     lane, so the 8 words of one value and row lie next to each other
 //     (68, not 64: 16 lanes' 16-byte reads then meet distinct banks). Lane
-//     4 q + p (q < 10) reads value q's 8 words of row p, adds them, and two
-//     quad_perm adds leave value q's 64-lane total in the quad's four lanes.
+//     4 q + p (q < 10) reads value q's 8 words of row p and adds them: value
+//     q's total of group p, which it adds to the sums of the key that the
+//     group visited.
 // Why LDS: on gfx950 a DPP add, a select or a compare issues in ~4.2 cycles
 // per wave and SIMD, a plain add, multiply or FMA in ~2.4, a permlane swap in
-// ~8.1 (measured, independent chains, 8 waves per SIMD), and the raster's LDS
-// pipe is mostly idle. Step 1 as DPP and the rest in LDS costs ~67 issue
-// cycles per visit; the lane-exchange network it replaces (DPP row halvings
-// per visit, then selects, quad_perms and swaps per pair of visits) ~110.
+// ~8.1 (measured, independent chains, 8 waves per SIMD). Lane exchanges for
+// all steps cost about 110 issue cycles per visit, this about 60.
 // Leaving step 1 to LDS as well would take half as many cycles again, but
 // would fill the LDS pipe. The matrix cores don't help: an MFMA holds the
 // SIMD's vector issue for its whole time (16-32 cycles) here.
@@ -409,11 +440,6 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
 // active (every branch of the visit loop is wave-uniform, and every wave of a
 // block is full): a DPP add whose source lane were inactive would leave its
 // output unwritten.
-template <int kCtrl>
-__device__ __forceinline__ uint32_t dpp(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xf, 0xf, false);
-}
-
 template <typename T>
 __device__ __forceinline__ uint32_t as_u(T v) { return __builtin_bit_cast(uint32_t, v); }
 template <typename T>
@@ -450,19 +476,19 @@ __device__ __forceinline__ void row_halve(const T* v, T* h5) {
 #undef GS_DPP_M
 
 // A wave's reduction scratch (5 rows of 64 words at red): where lane l writes
-// and reads, and the slot of the accumulator row it adds to (lane 4 q: q).
+// and reads, and the slot of the sums it adds to (lane 4 q + p: q).
 template <typename T>
 struct WaveRed {
   T* wr;
   const T* rd;
-  int slot;        // this lane's quad's value, clamped to 9
-  bool flusher;    // lane 4 q, q < 10
+  int slot;        // the value this lane sums and adds, clamped to 9
+  bool flusher;    // lane 4 q + p, q < 10
   __device__ __forceinline__ WaveRed(float4* red, int lane) {
     const int q = lane >> 2, qc = q < 10 ? q : 9;
     wr = reinterpret_cast<T*>(red) + lane;
     rd = reinterpret_cast<const T*>(red) + kRedStride * (qc % 5) + 16 * (lane & 3) + 8 * (qc / 5);
     slot = qc;
-    flusher = q < 10 && (lane & 3) == 0;
+    flusher = q < 10;
   }
   __device__ __forceinline__ void write(const T* h5) const {
 #pragma unroll
@@ -473,25 +499,22 @@ struct WaveRed {
     w8[0] = from_u<T>(a.x); w8[1] = from_u<T>(a.y); w8[2] = from_u<T>(a.z); w8[3] = from_u<T>(a.w);
     w8[4] = from_u<T>(b.x); w8[5] = from_u<T>(b.y); w8[6] = from_u<T>(b.z); w8[7] = from_u<T>(b.w);
   }
-  // the 64-lane total of this lane's slot, from its quad's words
+  // the 16-lane total of this lane's slot in group lane & 3
   __device__ __forceinline__ T total(const T* w8) const {
-    T s = ((w8[0] + w8[1]) + (w8[2] + w8[3])) + ((w8[4] + w8[5]) + (w8[6] + w8[7]));
-    s = s + from_u<T>(dpp<0xB1>(as_u(s)));
-    return s + from_u<T>(dpp<0x4E>(as_u(s)));
+    return ((w8[0] + w8[1]) + (w8[2] + w8[3])) + ((w8[4] + w8[5]) + (w8[6] + w8[7]));
   }
 };
 
-// Adds a visit's wave totals to Gaussian g's accumulator row (the flushing
-// lanes; zeros skipped). The asm keeps the total's last add ahead of the
-// branch, where it stays one DPP add.
+// Adds a visit's group totals to the batch's sums in LDS (the flushing
+// lanes). The asm keeps the reads of the words ahead of the branch, where
+// nothing waits for them yet.
 template <int kAccum, typename T>
-__device__ __forceinline__ void flush_sum(void* accum, uint32_t g, int slot, T r, bool flusher) {
+__device__ __forceinline__ void add_sum(T* sum, int key, int slot, T r, bool flusher) {
   asm volatile("" : "+v"(r));
-  if constexpr (kAccum == 0) {
-    if (flusher && r != 0u) atomicAdd((uint32_t*)accum + (int64_t)g * 12 + slot, r);
-  } else {
-    if (flusher && r != 0.0f) unsafeAtomicAdd((float*)accum + (int64_t)g * 12 + slot, r);
-  }
+  if (!flusher) return;
+  T* p = reinterpret_cast<T*>(reinterpret_cast<char*>(sum) + (__umul24((uint32_t)key, 40u) + 4u * (uint32_t)slot));
+  if constexpr (kAccum == 0) atomicAdd(p, r);
+  else unsafeAtomicAdd(p, r);
 }
 
 // kClampColour false: dL/dC is bounded (the Charbonnier loss: |dL/dC| <=
@@ -503,12 +526,18 @@ template <class S, int kAccum, bool kClampColour>
 __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, const RasterBufs& b, void* accum,
                                                 int tile, float4* lds, const PixelState* in = nullptr) {
   // three 16-byte records per staged splat, all at one index: one LDS address
+  constexpr int kKeys = RasterLds<S>::kKeys, kWords = S::kWaves * kGroups;
+  constexpr int kPart = kKeys / S::kWaves;   // keys that a wave stages and flushes
+  static_assert(kKeys / 64 * kGroups <= 64 && kWords <= 64, "one lane per chunk and group, and per block");
+  static_assert(kKeys <= 256 && (kPart % 64 == 0 || 64 % kPart == 0), "list entries are bytes; a part lies in a chunk");
   float4* const sA = lds;              // mx, my, A, B
-  float4* const sB = lds + S::B;       // C, opa*comp, -0.5 cnorm, id (bits)
-  float4* const sC = lds + 2 * S::B;   // r, g, b, opa
-  float4* const sRed = lds + 3 * S::B;
-  uint64_t (*const sMask)[S::kWaves] = reinterpret_cast<uint64_t (*)[S::kWaves]>(sRed + RasterLds<S>::kRed);
-  uint32_t& sEnd = *reinterpret_cast<uint32_t*>(&sMask[S::kChunks][0]);
+  float4* const sB = lds + (kKeys + 1);       // C, opa*comp, -0.5 cnorm, id (bits)
+  float4* const sC = lds + 2 * (kKeys + 1);   // r, g, b, opa
+  float4* const sRed = lds + 3 * (kKeys + 1);
+  uint8_t* const sList = reinterpret_cast<uint8_t*>(sRed + RasterLds<S>::kRed);
+  using AccT = typename std::conditional<kAccum == 0, uint32_t, float>::type;
+  AccT* const sSum = reinterpret_cast<AccT*>(sRed + RasterLds<S>::kRed + RasterLds<S>::kLists);   // 10 per key
+  uint32_t& sEnd = *reinterpret_cast<uint32_t*>(sSum + 10 * (kKeys + 1));
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
   const PixelMap pm = pixel_of_thread<S>(cam, tile, tid);
   const int x = pm.x, y = pm.y;
@@ -525,13 +554,16 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
   // The words of the last visit wait in the wave's scratch until the next
   // visit (or the end of the tile); before the first visit they are zeros,
   // which add nothing.
-  using AccT = typename std::conditional<kAccum == 0, uint32_t, float>::type;
   const WaveRed<AccT> red(sRed + wv * (5 * kRedStride / 4), lane);
   {
     const AccT z[5] = {};
     red.write(z);
   }
-  uint32_t lastGid = 0;
+  for (int k = wv * 10 * kPart + lane; k < (wv + 1) * 10 * kPart; k += 64) sSum[k] = AccT(0);
+  int lastKey = 0;                           // of the group this lane adds for
+  const int keyFrom = 4 * 16 * (lane & 3);   // a lane of it, as ds_bpermute counts
+  const int grp = lane >> 4;
+  uint8_t* const list = sList + (wv * kGroups + grp) * kKeys;
   float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float Ta = 0.0f;
   uint32_t myEnd = s;
@@ -548,7 +580,10 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
       myEnd = b.end[pi];
     }
   }
-  if (tid == 0) sEnd = s;
+  if (tid == 0) {
+    sEnd = s;
+    sA[kKeys] = sB[kKeys] = sC[kKeys] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);   // alpha 0: no lane takes it
+  }
   __syncthreads();
   if (myEnd > s) atomicMax(&sEnd, myEnd);
   __syncthreads();
@@ -569,59 +604,96 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
   const float gCs[3] = {gC[0] * kS, gC[1] * kS, gC[2] * kS};
   // 16384 dot(gC, S) of the colour-behind sum S, which enters only through it
   float GS = fmaf(gCs[2], cam.bg[2], fmaf(gCs[1], cam.bg[1], gCs[0] * cam.bg[0])) * Ta;
-  // batches start at multiples of S::B keys from s, as the forward's do, so
-  // that their chunks are the forward's chunks
+  // this wave's part of the last batch's sums to the Gaussians' accumulators
+  const auto flush = [&]() {
+#pragma unroll 1
+    for (int k = 10 * kPart * wv + lane; k < 10 * kPart * (wv + 1); k += 64) {
+      const AccT v = sSum[k];
+      if (v != AccT(0)) {
+        sSum[k] = AccT(0);
+        const uint32_t key = __umul24((uint32_t)k, 6554u) >> 16;   // k / 10 for k < 16384
+        const uint32_t id = __float_as_uint(sB[key].w);
+        AccT* row = (AccT*)accum + (uint64_t)id * 12;
+        if constexpr (kAccum == 0) atomicAdd(row + ((uint32_t)k - __umul24(key, 10u)), v);
+        else unsafeAtomicAdd(row + ((uint32_t)k - __umul24(key, 10u)), v);
+      }
+    }
+  };
+  // batches start at multiples of 64 keys from s, so that their chunks are
+  // the forward's chunks
   for (uint32_t hi = endMax; hi > s; ) {
-    const uint32_t lo = s + (hi - s - 1u) / S::B * S::B;
+    const uint32_t lo = s + (hi - s - 1u) / kKeys * kKeys;
     const int n = (int)(hi - lo);
-    __syncthreads();
-    for (int c = wv; c < S::kChunks && 64 * c < n; c += S::kWaves) {
-      // key 64 c + l goes to record 64 c + 63 - l, so that the walk towards the
-      // first key is an ascending one (find-first-bit on the reversed mask)
-      const int j = 64 * c + lane, r = 64 * c + 63 - lane;
-      const uint64_t* tw = b.took + took_word<S>(s, tile, ((lo - s) >> 6) + (uint32_t)c);
-      if (lane < S::kWaves) sMask[c][lane] = tw[lane];
-      uint64_t any = 0ull;   // keys that some wave of the tile took: only these are loaded
-#pragma unroll
-      for (int w = 0; w < S::kWaves; w++) any |= tw[w];
-      if (j < n && ((any >> lane) & 1ull) != 0ull) {
+    // lane 4 c + q: this wave's word of chunk c and group q (those of chunks
+    // that the wave did not reach may be stale)
+    const uint32_t first = lo + 64u * (uint32_t)(lane / kGroups);   // the chunk's first key
+    uint64_t words = 0ull;
+    if (lane < kKeys / 64 * kGroups && first < waveEnd) {
+      words = b.took[took_word<S>(s, tile, ((lo - s) >> 6) + (uint32_t)(lane / kGroups)) + wv * kGroups + lane % kGroups];
+      if (waveEnd - first < 64u) words &= (1ull << (waveEnd - first)) - 1ull;
+    }
+    __syncthreads();   // the last batch's visits are done
+    if (hi != endMax) flush();
+#pragma unroll 1
+    for (int p0 = wv * kPart; p0 < (wv + 1) * kPart && p0 < n; p0 += 64) {
+      const int j = p0 + lane;
+      const uint64_t* tw = b.took + took_word<S>(s, tile, ((lo - s) >> 6) + (uint32_t)(p0 >> 6));
+      const uint64_t word = lane < kWords ? tw[lane] : 0ull;
+      // keys that some block of the tile took: only these are loaded
+      const uint64_t any = ((uint64_t)or_lanes<kWords>((uint32_t)(word >> 32)) << 32) | or_lanes<kWords>((uint32_t)word);
+      if (lane < kPart && j < n && ((any >> (j & 63)) & 1ull) != 0ull) {
         const uint32_t id = b.ids[lo + (uint32_t)j] & kIdMask;
         if (b.recFmt == 0) {
           const float4 r1 = b.rec[4 * id + 1];
-          sA[r] = b.rec[4 * id + 0];
-          sC[r] = b.rec[4 * id + 2];
-          sB[r] = make_float4(r1.x, r1.y, b.rec[4 * id + 3].y, __uint_as_float(id));
+          sA[j] = b.rec[4 * id + 0];
+          sC[j] = b.rec[4 * id + 2];
+          sB[j] = make_float4(r1.x, r1.y, b.rec[4 * id + 3].y, __uint_as_float(id));
         } else {
           const float4 r1 = b.rec[3 * id + 1];
           const float4 d = b.rec[3 * id + 2];   // comp, -0.5 cnorm, 1 - opa, opa
-          sA[r] = b.rec[3 * id + 0];
-          sC[r] = record_colour(b.recFmt, r1, d.w);
-          sB[r] = make_float4(r1.x, r1.y, d.y, __uint_as_float(id));
+          sA[j] = b.rec[3 * id + 0];
+          sC[j] = record_colour(b.recFmt, r1, d.w);
+          sB[j] = make_float4(r1.x, r1.y, d.y, __uint_as_float(id));
         }
       }
     }
     __syncthreads();
-    for (int c = S::kChunks - 1; c >= 0; c--) {
-      const uint32_t g0 = lo + 64u * (uint32_t)c;   // key of bit 0
-      if (waveEnd <= g0) continue;                  // no lane got this far: the words may be stale
-      uint64_t m = uniform64(sMask[c][wv]);
-      if (waveEnd - g0 < 64u) m &= (1ull << (waveEnd - g0)) - 1ull;
-      m = __builtin_bitreverse64(m);
-      // record r of the chunk is key g0 + 63 - r: before this lane's end when
-      // r is above pastEnd
-      const int pastEnd = (int)(g0 + 63u - myEnd);
-      while (m) {
-        const int bit = (int)__builtin_ctzll(m);
-        clear_bit(m, bit);
+    const int pastEnd = (int)(myEnd - lo);   // this lane's end as an index of the batch
+    // each group's keys, last one first, then the record that nobody takes
+    constexpr uint32_t kNone = 0x01010101u * (uint32_t)kKeys;
+    int have[kGroups] = {};
+    for (int k = lane; k < kGroups * kKeys / 8; k += 64)
+      reinterpret_cast<uint2*>(sList + wv * kGroups * kKeys)[k] = make_uint2(kNone, kNone);
+#pragma unroll
+    for (int c = kKeys / 64 - 1; c >= 0; c--) {
+#pragma unroll
+      for (int q = 0; q < kGroups; q++) {
+        const uint32_t mLo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)words, kGroups * c + q);
+        const uint32_t mHi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(words >> 32), kGroups * c + q);
+        const uint64_t m = ((uint64_t)mHi << 32) | mLo;
+        const int cnt = __builtin_popcountll(m);
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(mHi, __builtin_amdgcn_mbcnt_lo(mLo, 0u));
+        if (__builtin_amdgcn_inverse_ballot_w64(m))
+          list[kKeys * (q - grp) + have[q] + cnt - 1 - (int)below] = (uint8_t)(64 * c + lane);
+        have[q] += cnt;
+      }
+    }
+    const int steps = max(max(have[0], have[1]), max(have[2], have[3]));
+    if (steps != 0) {
+      int nextKey = (int)list[0];
+      for (int step = 0; step < steps; step++) {
         // Straight-line for all 64 lanes; lanes that do not take the splat
         // (outside the image, past their `end`, outside the cutoff, alpha
-        // below A_MIN) keep their state and contribute zero terms. Some
-        // lane took the splat in the forward, so there is nothing to vote on.
+        // below A_MIN, their group past its list) keep their state and
+        // contribute zero terms. Some lane of the group took the splat in the
+        // forward, so there is nothing to vote on.
         AccT w8[8];
         red.read(w8);   // the previous visit's words
-        const uint32_t jo = lds_offset((uint32_t)bit * 16u);
-        const float4 a = lds_at<float4>(sA + 64 * c, jo);
-        const float4 bb = lds_at<float4>(sB + 64 * c, jo);   // C, opa*comp, -0.5 cnorm, id
+        const int key = nextKey;
+        nextKey = (int)list[step + 1 < kKeys ? step + 1 : 0];
+        const uint32_t jo = (uint32_t)key * 16u;
+        const float4 a = lds_at<float4>(sA, jo);
+        const float4 bb = lds_at<float4>(sB, jo);   // C, opa*comp, -0.5 cnorm, id
         const float dx = px - a.x, dy = py - a.y;
         const float cA = a.z, cB = a.w, cC = bb.x;
         const float t2 = fmaf(cC * dy, dy, (cA * dx) * dx);
@@ -630,8 +702,8 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
         const float G = gs_expf_raster(-e);
         const float araw = bb.y * G;
         const float alpha = fminf(0.99f, araw);
-        const bool contrib = bit > pastEnd && e <= cut.eCut && alpha >= cut.aMin;
-        const float4 c4 = lds_at<float4>(sC + 64 * c, jo);
+        const bool contrib = key < pastEnd && e <= cut.eCut && alpha >= cut.aMin;
+        const float4 c4 = lds_at<float4>(sC, jo);
         // Tb = Ta / (1 - alpha), S / (1 - alpha) through one reciprocal.
         // 1 - alpha lies in [0.0099, 1] (alpha in [0, 0.99]); on [2^-9, 1]
         // v_rcp_f32 refined by one FMA Newton step equals the correctly
@@ -641,6 +713,7 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
         const float alphaE = contrib ? alpha : 0.0f;
         const float rom = rcp_exact_unit(1.0f - alphaE);
         const float Tb = Ta * rom;
+        add_sum<kAccum>(sSum, lastKey, red.slot, red.total(w8), red.flusher);
         const float gcol = fmaf(gCs[2], c4.z, fmaf(gCs[1], c4.y, gCs[0] * c4.x));   // scaled
         // Every term is a product with galpha or aT, which are zero for the
         // lanes that do not take the splat (all other factors are finite).
@@ -682,18 +755,25 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
 #pragma unroll
           for (int q = 0; q < 10; q++) cur[q] = v[q];
         }
+        // the next key has arrived by now: waited for here, not behind the
+        // writes below
+        asm volatile("" : "+v"(nextKey));
         AccT h[5];
         row_halve<AccT>(cur, h);
-        flush_sum<kAccum>(accum, lastGid, red.slot, red.total(w8), red.flusher);
         red.write(h);
-        lastGid = __float_as_uint(bb.w);
+        lastKey = __builtin_amdgcn_ds_bpermute(keyFrom, key);
       }
     }
+    // the last visit's words, while its batch is staged
+    AccT w8[8];
+    red.read(w8);
+    add_sum<kAccum>(sSum, lastKey, red.slot, red.total(w8), red.flusher);
+    const AccT z[5] = {};
+    red.write(z);
     hi = lo;
   }
-  AccT w8[8];
-  red.read(w8);
-  flush_sum<kAccum>(accum, lastGid, red.slot, red.total(w8), red.flusher);
+  __syncthreads();
+  if (endMax > s) flush();
 }
 
 template <class S, int kLoss>
@@ -703,7 +783,7 @@ __global__ __launch_bounds__(S::kThreads) void k_raster_fwd(Cam cam, Cut cut, Ra
 }
 
 template <class S, int kAccum, bool kClampColour>
-__global__ __launch_bounds__(S::kThreads) void k_raster_bwd(Cam cam, Cut cut, RasterBufs b, void* accum) {
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::kBwdWavesPerEU))) void k_raster_bwd(Cam cam, Cut cut, RasterBufs b, void* accum) {
   __shared__ float4 lds[RasterLds<S>::kBwd];
   raster_bwd_tile<S, kAccum, kClampColour>(cam, cut, b, accum, tile_of_block(b), lds);
 }
@@ -714,7 +794,7 @@ __global__ __launch_bounds__(S::kThreads) void k_raster_bwd(Cam cam, Cut cut, Ra
 // keeps its pixel's T, end and dL/dC in registers; they are stored too,
 // for the debug readbacks).
 template <class S, int kAccum, bool kClampColour>
-__global__ __launch_bounds__(S::kThreads) void k_raster_fwd_bwd(Cam cam, Cut cut, RasterBufs b, void* accum) {
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::kBwdWavesPerEU))) void k_raster_fwd_bwd(Cam cam, Cut cut, RasterBufs b, void* accum) {
   __shared__ float4 lds[RasterLds<S>::kBoth];   // the two passes' layouts share it
   const int tile = tile_of_block(b);
   PixelState ps;
@@ -775,7 +855,7 @@ k_raster_fwd_bwd_views(const ViewBlock* __restrict__ vb, Cut cut, uint32_t* queu
 // one view of a batched step, one block per tile (camera and buffers from
 // device memory), forward with the loss and backward in one launch
 template <class S, int kAccum, bool kClampColour>
-__global__ __launch_bounds__(S::kThreads) void k_raster_fwd_bwd_view(const ViewBlock* __restrict__ vb, int v,
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::kBwdWavesPerEU))) void k_raster_fwd_bwd_view(const ViewBlock* __restrict__ vb, int v,
                                                                      Cut cut) {
   const Cam cam = vb->cams[v];
   const RasterBufs b = global_bufs(vb->bufs[v]);
@@ -803,11 +883,11 @@ static void with_shape(const RasterShape& sh, F&& f) {
 }
 
 size_t raster_took_bytes(int w, int h, int64_t keys) {
-  // took_word's last row at each tile size: one word per wave (tile^2 / 64)
+  // took_word's last row at each tile size: one word per 4x4 pixels
   size_t words = 0;
   for (int t = 8; t <= 32; t *= 2) {
     const size_t tiles = (size_t)((w + t - 1) / t) * (size_t)((h + t - 1) / t);
-    const size_t need = ((size_t)keys / 64 + tiles + 1) * (size_t)(t * t / 64);
+    const size_t need = ((size_t)keys / 64 + tiles + 1) * (size_t)(t * t / 16);
     words = words > need ? words : need;
   }
   return words * 8;

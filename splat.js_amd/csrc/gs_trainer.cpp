@@ -119,7 +119,7 @@ struct gs_trainer {
   float* Tfin = nullptr;
   uint32_t* endIdx = nullptr;
   float4* gC = nullptr;
-  uint64_t* took = nullptr;      // the training forward's taken keys per wave (RasterBufs::took)
+  uint64_t* took = nullptr;      // the training forward's taken keys (RasterBufs::took)
   float* ssimScratch = nullptr;  // 9 x maxPix SSIM partials (L1 + D-SSIM loss only)
   uint32_t* targets = nullptr;
   int64_t totalPx = 0;

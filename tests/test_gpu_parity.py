@@ -691,3 +691,36 @@ def test_view_read_in_blocks(W, H):
     t.destroy()
     for v in (a, b):
         np.testing.assert_array_equal(v.reshape(-1).view(np.uint32), ref.reshape(-1).view(np.uint32))
+
+
+@pytest.mark.parametrize("tile,batch", [(16, 256), (16, 64), (32, 256), (8, 128)])
+@pytest.mark.parametrize("n", [1, 63, 65, 127, 128, 129, 257, 385])
+def test_backward_lists_at_the_edges_of_their_batches(n, tile, batch):
+    """One view of 24x16 pixels: n faint splats, half of them inside one 4x4
+    block, half over the whole view, so that the groups of a wave have lists
+    of different lengths (none among them), over one batch of 128 keys, one
+    key more or less, and several. Bit-exact against the restatement."""
+    print(n, tile, batch, flush=True)
+    rng = np.random.default_rng(n)
+    W, H, f = 24, 16, 24.0
+    p = np.zeros((n, 16), np.float32)
+    z = rng.uniform(2.0, 4.0, n)
+    wide = rng.random(n) < 0.5
+    p[:, 0] = rng.uniform(-0.5, 0.5, n) * W / f * z
+    p[:, 1] = rng.uniform(-0.5, 0.5, n) * H / f * z
+    p[:, 2] = z
+    p[:, 3:6] = np.where(wide, np.log(1.0), np.log(0.02))[:, None] + rng.normal(0, 0.1, (n, 3))
+    p[:, 6] = 1.0
+    p[:, 10:13] = rng.normal(0, 1, (n, 3))
+    p[:, 13] = np.where(wide, -4.0, -1.0)
+    cams = [{"imgIdx": 0, "R": [1, 0, 0, 0, 1, 0, 0, 0, 1], "t": [0, 0, 0], "f": f, "cx": W / 2, "cy": H / 2, "w": W, "h": H}]
+    images = [{"tw": W, "th": H, "rgb": rng.random((H * W, 3)).astype(np.float32)}]
+    t = _trainer(p, None, cams, images, W, H, 1.0, {}, shDeg=0, tile=tile, batch=batch)
+    t.iter = 5000
+    ref = OracleTrainer(p, None, cams, images, 1.0, opts={}, shDeg=0, tile=tile)
+    ref.iter = 5000
+    g, r = t.step_debug(0), ref.step(0)
+    out = t.readGaussians()
+    t.destroy()
+    np.testing.assert_array_equal(g["accum"], r["accum"])
+    np.testing.assert_array_equal(out["data"].view(np.uint32), ref.P.view(np.uint32))
