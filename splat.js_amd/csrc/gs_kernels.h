@@ -322,6 +322,10 @@ struct RefineOp {
 };
 
 // q[i] = (opacity logit, log-scale x, y, z) for i < n
+// Copies the statistics src to out (pinned), clears window's loss sums, src too
+// where clearSrc, and camWords words of camGrad.
+void launch_stats_read(hipStream_t st, double* src, double* window, double* out, bool clearSrc, uint32_t* camGrad,
+                       int64_t camWords);
 // Rows [first, first + count) of the parameters (16 floats each) and of the SH
 // coefficients (C floats each; fmt 0 f32 planes, 1 bf16, 2 fp16) into out.
 void launch_param_rows(hipStream_t st, int64_t cap, int64_t first, int64_t count, const float4* P, float* out);

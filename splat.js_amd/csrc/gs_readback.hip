@@ -1,5 +1,5 @@
-// gs_readback.hip — the Gaussians in the caller's layout (readGaussians,
-// trainer.js:797-817): 16 floats and 3K coefficients per row, from the
+// gs_readback.hip — what the host reads: the statistics of a loss or PSNR read,
+// and the Gaussians in the caller's layout (readGaussians, trainer.js:797-817): 16 floats and 3K coefficients per row, from the
 // 16-byte planes, written over PCIe straight into pinned host memory.
 //
 // The device lays the rows out and decodes 16-bit coefficients, so that the
@@ -31,6 +31,25 @@ __global__ __launch_bounds__(kBlock) void k_sh_rows(int64_t cap, int64_t first, 
     const uint32_t b = ((const uint16_t*)SH)[((j >> 3) * cap + first + r) * 8 + (j & 7u)];
     out[k] = kFmt == 2 ? gs_h2f(b) : gs_bf2f(b);
   }
+}
+
+// One block: the statistics src into pinned memory, the loss window cleared
+// (all but its dropped keys), and with a PSNR read also src and the camera
+// gradient rows. What a copy and up to three memsets did in launches of their
+// own, some 3 us each: four evaluated 979x546 views 469 -> 439 us.
+__global__ __launch_bounds__(1024) void k_stats_read(double* src, double* window, double* __restrict__ out, bool clearSrc,
+                                                     uint32_t* __restrict__ camGrad, int64_t camWords) {
+  for (int i = threadIdx.x; i < kStatDoubles; i += 1024) {
+    out[i] = src[i];
+    if (clearSrc) src[i] = 0.0;
+    if (i < kStatDropped) window[i] = 0.0;   // the same thread read it above where it is src
+  }
+  for (int64_t i = threadIdx.x; i < camWords; i += 1024) camGrad[i] = 0u;
+}
+
+void launch_stats_read(hipStream_t st, double* src, double* window, double* out, bool clearSrc, uint32_t* camGrad,
+                       int64_t camWords) {
+  k_stats_read<<<1, 1024, 0, st>>>(src, window, out, clearSrc, camGrad, camWords);
 }
 
 void launch_param_rows(hipStream_t st, int64_t cap, int64_t first, int64_t count, const float4* P, float* out) {

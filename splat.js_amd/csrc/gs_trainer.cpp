@@ -125,6 +125,7 @@ struct gs_trainer {
   int64_t totalPx = 0;
   double* stats = nullptr;      // training stats (kStatDoubles)
   double* evalStats = nullptr;  // eval/view stats (kStatDoubles)
+  bool evalClean = false;       // evalStats is zero once the stream's work so far is done
   uint32_t* camGrad = nullptr;  // (numCams + 1) x 8 i32 camera gradient rows (trainer.js:173)
 
   std::vector<CamMeta> cams;
@@ -470,6 +471,7 @@ void radix_values_into(BinArgs& a, uint32_t* ids, uint32_t* scratch) {
 // ---- one raster: project -> bin/sort -> forward (+ loss) ----
 int run_raster(gs_trainer* h, const Cam& cam, int loss, double* statsBuf, bool withBwd = false) {
   const int64_t n = h->n;
+  if (statsBuf == h->evalStats) h->evalClean = false;
   h->lastViews = 0;
   h->profLast = nullptr;   // a step or render starts its own first stage
   {
@@ -998,6 +1000,7 @@ int enqueue_views(gs_trainer* h, const ViewBlock& vb, gs_debug_out* dbg, float* 
 // raster statistics to statsBuf) and appends the step's shape to key.
 int fill_views(gs_trainer* h, const int* ci, int count, int activeDeg, double* statsBuf, ViewBlock& vb,
                std::vector<int64_t>& key) {
+  if (statsBuf == h->evalStats) h->evalClean = false;
   memset(&vb, 0, sizeof vb);
   vb.count = count;
   uint32_t off = 0;
@@ -1876,8 +1879,8 @@ int gs_read_loss_async(gs_trainer_t* h, gs_pending_t** out) {
   if (rc != GS_OK) return rc;
   // copy the window's stats, then reset the window; the budget drops behind
   // it keep counting across windows (trainer.js:621-627)
-  hipError_t e = hipMemcpyAsync(p->stats, h->stats, 8 * kStatDoubles, hipMemcpyDeviceToHost, h->st);
-  if (e == hipSuccess) e = hipMemsetAsync(h->stats, 0, 8 * kStatDropped, h->st);
+  launch_stats_read(h->st, h->stats, h->stats, p->stats, false, nullptr, 0);
+  hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipEventRecord(p->ev, h->st);
   if (e != hipSuccess) {
     gs_pending_free(p);
@@ -1898,17 +1901,17 @@ int gs_eval_cam_psnr_async(gs_trainer_t* h, int32_t ci, gs_pending_t** out) {
   const CamMeta& m = h->cams[ci];
   // the reference evaluates with the camera's training uniform (trainer.js:547)
   const Cam cam = make_cam_meta(h, m, m.activeDeg);
-  HIPCK(hipMemsetAsync(h->evalStats, 0, 8 * kStatDoubles, h->st));
+  if (!h->evalClean) HIPCK(hipMemsetAsync(h->evalStats, 0, 8 * kStatDoubles, h->st));
   int rc = run_raster(h, cam, 1, h->evalStats);
   if (rc) return rc;
   gs_pending* p = nullptr;
   rc = pending_new(h, gs_pending::kPsnr, &p);
   if (rc != GS_OK) return rc;
-  hipError_t e = hipMemcpyAsync(p->stats, h->evalStats, 8 * kStatDoubles, hipMemcpyDeviceToHost, h->st);
   // trainer.js:562, :570-571: the camera gradient rows are drained and the
   // training loss window is reset too
-  if (e == hipSuccess) e = hipMemsetAsync(h->camGrad, 0, (h->cams.size() + 1) * 32, h->st);
-  if (e == hipSuccess) e = hipMemsetAsync(h->stats, 0, 8 * kStatDropped, h->st);
+  launch_stats_read(h->st, h->evalStats, h->stats, p->stats, true, h->camGrad, (int64_t)(h->cams.size() + 1) * 8);
+  hipError_t e = hipGetLastError();
+  h->evalClean = e == hipSuccess;
   if (e == hipSuccess) e = hipEventRecord(p->ev, h->st);
   if (e != hipSuccess) {
     gs_pending_free(p);

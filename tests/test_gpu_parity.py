@@ -724,3 +724,20 @@ def test_backward_lists_at_the_edges_of_their_batches(n, tile, batch):
     t.destroy()
     np.testing.assert_array_equal(g["accum"], r["accum"])
     np.testing.assert_array_equal(out["data"].view(np.uint32), ref.P.view(np.uint32))
+
+
+def test_psnr_reads_start_from_cleared_statistics():
+    """A PSNR read leaves its statistics cleared for the next one; a training
+    view rendered in between adds to them. The sums' atomics come in any
+    order, in f64: 1e-9 relative."""
+    p, sh, cams, images, W, H, radius = config1_setup(n=3000)
+    t = _trainer(p, sh, cams, images, W, H, radius, {}, shDeg=2)
+    first = t.evalCamPsnr(0)
+    again = t.evalCamPsnr(0)
+    t.renderView(t.camMeta[0], 1, t.camMeta[0]["offset"])
+    after = t.evalCamPsnr(0)
+    t.stepOnce(0)
+    assert t.readLoss() > 0.0
+    assert t.readLoss() is None
+    t.destroy()
+    np.testing.assert_allclose([again, after], first, rtol=1e-9)
