@@ -27,24 +27,31 @@
 // its pixels down to the first key (each wave from the largest `end` of its
 // own pixels), recomputing each pixel's transmittance
 // in front of a splat from the stored final T (Tb = Ta/(1-a), through one
-// reciprocal that also scales the colour-behind sum S). The 16-lane groups of
-// a wave (4x4 pixels each) walk lists of their own: the keys that some lane
-// of the group took in the forward, which leaves one word per 64 keys and
-// group for this (RasterBufs::took). A wave is done with a batch of 128 keys
-// when its longest list is: a splat that misses a group costs it nothing,
-// where a walk of the whole wave's keys left half of the lanes idle.
-// Per visit, the 10 screen-space gradient terms of each group's 16 pixels are
-// summed (one DPP step, then the wave's own LDS scratch; WaveRed below) and
-// added to the batch's sums in LDS; these go to the Gaussians' accumulators
-// with one atomic per key, term and tile once the batch is done:
-//   GS_ACCUM_FIXED: each pixel's term is converted to i32 first,
+// reciprocal that also scales the colour-behind sum S). It visits the keys
+// that some lane took in the forward, which leaves words of 64 keys for this
+// (RasterBufs::took). Per visit, the 10 screen-space gradient terms are summed
+// over lanes (one DPP step, then the wave's own LDS scratch; WaveRed below).
+//   GS_ACCUM_FIXED: the 16-lane groups of a wave (4x4 pixels each) walk lists
+//                   of their own, from a word per group. A wave is done with a
+//                   batch of 128 keys when its longest list is: a splat that
+//                   misses a group costs it nothing, where a walk of the whole
+//                   wave's keys left half of the lanes idle. The groups' sums
+//                   are added to the batch's sums in LDS; these go to the
+//                   Gaussians' accumulators with one atomic per key, term and
+//                   tile once the batch is done.
+//                   Each pixel's term is converted to i32 first,
 //                   i32(clamp(v * 16384, -1e9, 1e9)), exactly as the
 //                   reference's atomicAdd on atomic<i32> (shaders.js:529-541);
 //                   integer sums commute, so the result is deterministic and
 //                   bit-identical to any other summation order. (Under the
 //                   Charbonnier loss the three colour terms cannot reach the
 //                   clamp and convert without it.)
-//   GS_ACCUM_F32:   plain f32 sums (atomic add order is not deterministic).
+//   GS_ACCUM_F32:   plain f32 sums (atomic add order is not deterministic). A
+//                   wave walks its keys as one, and adds its 64 pixels' sums
+//                   to the Gaussian's accumulator with one atomic per term: a
+//                   float added in LDS costs several times an integer one, so
+//                   the groups' lists took 1160 us where this takes 666 (1M
+//                   Gaussians at 1600x900, forward and backward).
 //
 // Training under the Charbonnier loss runs both passes in one launch: the
 // loss gradient of a pixel needs only that pixel, so a block runs its tile's
@@ -58,8 +65,8 @@
 // where the chip is full, and on small images, with about one wave per SIMD,
 // every instruction, scalar ones included (~4 cycles each there). So the
 // masks of a forward visit live in scalar registers, with one instruction to
-// clear a bit. Backward with lists per group against a walk of the wave's
-// keys with an atomic per wave: 20k Gaussians at 320x240 87 -> 64 us, 600k at
+// clear a bit. Backward with lists per group (fixed-point sums) against a walk
+// of the wave's keys with an atomic per wave: 20k Gaussians at 320x240 87 -> 64 us, 600k at
 // 1237x933 389 -> 315; forward and backward in one launch, 160 Gaussians at
 // 64x64 28 -> 24, 123k at 737x411 93 -> 79, 1M at 1600x900 566 -> 543, 8 views
 // of 1M 3865 -> 3745. Where splats cover whole tiles the lists of a wave are
@@ -172,6 +179,12 @@ __device__ __forceinline__ void clear_bit(uint64_t& m, int bit) {
   asm("s_bitset0_b64 %0, %1" : "+s"(m) : "s"(bit));
 }
 
+// the same when `mask` is empty (left to the compiler: five instructions)
+__device__ __forceinline__ void clear_bit_if_none(uint64_t& m, int bit, uint64_t mask) {
+  asm("s_cmp_lg_u64 %1, 0\n\ts_cbranch_scc1 .Lgs_some%=\n\ts_bitset0_b64 %0, %2\n.Lgs_some%=:"
+      : "+s"(m) : "s"(mask), "s"(bit) : "scc");
+}
+
 // the OR over the first n lanes (the others hold 0), in a scalar register
 template <int n>
 __device__ __forceinline__ uint32_t or_lanes(uint32_t v) {
@@ -250,9 +263,11 @@ __device__ __forceinline__ size_t took_word(uint32_t s, int tile, uint32_t c) {
 
 // One tile of the forward pass, by the whole 256-thread block. The block's
 // threads must all call it (it synchronises), and nothing else may use the
-// block's LDS until every thread has returned. kTook: record the keys each
-// wave's lanes take, for the backward.
-template <class S, int kLoss, bool kTook>
+// block's LDS until every thread has returned. What the backward needs of the
+// keys that are taken: kTookGroups, each 16-lane group's; kTookWaves, each
+// wave's, as the word of its first group (a scalar word: no lane writes).
+constexpr int kTookNone = 0, kTookGroups = 1, kTookWaves = 2;
+template <class S, int kLoss, int kTook>
 __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, const RasterBufs& b, int tile,
                                                 float4* lds, PixelState* out = nullptr) {
   float4* const sA = lds;              // mx, my, A, B
@@ -305,7 +320,8 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
     if (run != 0ull) {
       for (int c = 0; c < S::kChunks; c++) {
         uint64_t m = uniform64(sMask[c][mslot]);
-        int tkLo = 0, tkHi = 0;   // kTook: lane k holds the lanes that take key k of the chunk
+        int tkLo = 0, tkHi = 0;   // kTookGroups: lane k holds the lanes that take key k of the chunk
+        uint64_t took = m;        // kTookWaves: the keys that some lane takes
         while (m) {
           const int bit = (int)__builtin_ctzll(m);
           clear_bit(m, bit);
@@ -322,10 +338,11 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
           // and the exp below needs its argument in [-87, 0]
           const float ee = clamp_e(fmaf(0.5f, t2, (a.w * dx) * dy));
           const uint64_t live = run & wave_ballot(ee <= cut.eCut);
+          uint64_t take = 0ull;
           if (live != 0ull) {
             const float araw = bb.y * gs_expf_raster(-ee);
             const float alpha = fminf(0.99f, araw);
-            const uint64_t take = live & wave_ballot(alpha >= cut.aMin);
+            take = live & wave_ballot(alpha >= cut.aMin);
             if (__builtin_amdgcn_inverse_ballot_w64(take)) {
               const float4 c4 = lds_at<float4>(sC + 64 * c, jo);
               const float w = T * alpha;
@@ -337,7 +354,7 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
             // T only falls here, so a lane reaches T < 1e-4 on this splat
             // exactly when it is still running and now below; that happens
             // once per pixel, so its bookkeeping sits behind a scalar branch
-            if (kTook) {
+            if (kTook == kTookGroups) {
               tkLo = write_lane((int)(uint32_t)take, bit, tkLo);
               tkHi = write_lane((int)(uint32_t)(take >> 32), bit, tkHi);
             }
@@ -348,8 +365,14 @@ __device__ __forceinline__ void raster_fwd_tile(const Cam& cam, const Cut& cut, 
               if (run == 0ull) m = 0ull;
             }
           }
+          if (kTook == kTookWaves) clear_bit_if_none(took, bit, take);
         }
-        if (kTook && 64u * (uint32_t)c < cnt) {
+        if (kTook == kTookWaves && 64u * (uint32_t)c < cnt && lane == 0) {
+          ulonglong2* tw = (ulonglong2*)(b.took + took_word<S>(s, tile, ((base - s) >> 6) + (uint32_t)c) + wv * kGroups);
+          tw[0] = make_ulonglong2(took, 0ull);
+          tw[1] = make_ulonglong2(0ull, 0ull);
+        }
+        if (kTook == kTookGroups && 64u * (uint32_t)c < cnt) {
           const uint64_t w0 = wave_ballot(((uint32_t)tkLo & 0xffffu) != 0u), w1 = wave_ballot(((uint32_t)tkLo >> 16) != 0u);
           const uint64_t w2 = wave_ballot(((uint32_t)tkHi & 0xffffu) != 0u), w3 = wave_ballot(((uint32_t)tkHi >> 16) != 0u);
           if (lane == 0) {
@@ -475,6 +498,12 @@ __device__ __forceinline__ void row_halve(const T* v, T* h5) {
 #undef GS_ROW_STEP
 #undef GS_DPP_M
 
+// x of the lane that a DPP quad permutation selects
+template <int kCtrl, typename T>
+__device__ __forceinline__ T quad(T x) {
+  return from_u<T>((uint32_t)__builtin_amdgcn_mov_dpp((int)as_u(x), kCtrl, 0xf, 0xf, false));
+}
+
 // A wave's reduction scratch (5 rows of 64 words at red): where lane l writes
 // and reads, and the slot of the sums it adds to (lane 4 q + p: q).
 template <typename T>
@@ -503,18 +532,29 @@ struct WaveRed {
   __device__ __forceinline__ T total(const T* w8) const {
     return ((w8[0] + w8[1]) + (w8[2] + w8[3])) + ((w8[4] + w8[5]) + (w8[6] + w8[7]));
   }
+  // the wave's total of this lane's slot, in the quad's four lanes
+  __device__ __forceinline__ T wave_total(const T* w8) const {
+    T s = total(w8);
+    s = s + quad<0xB1>(s);   // quad_perm [1,0,3,2]
+    return s + quad<0x4E>(s);   // quad_perm [2,3,0,1]
+  }
 };
 
-// Adds a visit's group totals to the batch's sums in LDS (the flushing
-// lanes). The asm keeps the reads of the words ahead of the branch, where
-// nothing waits for them yet.
-template <int kAccum, typename T>
-__device__ __forceinline__ void add_sum(T* sum, int key, int slot, T r, bool flusher) {
+// GS_ACCUM_FIXED: adds a visit's group totals to the batch's sums in LDS (the
+// flushing lanes). The asm keeps the reads of the words ahead of the branch,
+// where nothing waits for them yet.
+__device__ __forceinline__ void add_group_sums(uint32_t* sum, int key, int slot, uint32_t r, bool flusher) {
   asm volatile("" : "+v"(r));
   if (!flusher) return;
-  T* p = reinterpret_cast<T*>(reinterpret_cast<char*>(sum) + (__umul24((uint32_t)key, 40u) + 4u * (uint32_t)slot));
-  if constexpr (kAccum == 0) atomicAdd(p, r);
-  else unsafeAtomicAdd(p, r);
+  atomicAdd(reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(sum) + (__umul24((uint32_t)key, 40u) + 4u * (uint32_t)slot)), r);
+}
+
+// GS_ACCUM_F32: adds a visit's wave totals to Gaussian g's accumulator row (a
+// lane per slot; zeros skipped). The asm keeps the total's last add ahead of
+// the branch.
+__device__ __forceinline__ void add_wave_sums(float* accum, uint32_t g, int slot, float r, bool flusher) {
+  asm volatile("" : "+v"(r));
+  if (flusher && r != 0.0f) unsafeAtomicAdd(accum + (uint64_t)g * 12 + (uint32_t)slot, r);
 }
 
 // kClampColour false: dL/dC is bounded (the Charbonnier loss: |dL/dC| <=
@@ -559,9 +599,11 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
     const AccT z[5] = {};
     red.write(z);
   }
-  for (int k = wv * 10 * kPart + lane; k < (wv + 1) * 10 * kPart; k += 64) sSum[k] = AccT(0);
-  int lastKey = 0;                           // of the group this lane adds for
+  if constexpr (kAccum == 0)
+    for (int k = wv * 10 * kPart + lane; k < (wv + 1) * 10 * kPart; k += 64) sSum[k] = 0u;
+  int lastKey = 0;                           // fixed: of the group this lane adds for
   const int keyFrom = 4 * 16 * (lane & 3);   // a lane of it, as ds_bpermute counts
+  uint32_t lastId = 0;                       // f32: the Gaussian of the last visit
   const int grp = lane >> 4;
   uint8_t* const list = sList + (wv * kGroups + grp) * kKeys;
   float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -604,20 +646,101 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
   const float gCs[3] = {gC[0] * kS, gC[1] * kS, gC[2] * kS};
   // 16384 dot(gC, S) of the colour-behind sum S, which enters only through it
   float GS = fmaf(gCs[2], cam.bg[2], fmaf(gCs[1], cam.bg[1], gCs[0] * cam.bg[0])) * Ta;
-  // this wave's part of the last batch's sums to the Gaussians' accumulators
+  // fixed: this wave's part of the last batch's sums to the Gaussians' accumulators
   const auto flush = [&]() {
+    if constexpr (kAccum == 0) {
 #pragma unroll 1
-    for (int k = 10 * kPart * wv + lane; k < 10 * kPart * (wv + 1); k += 64) {
-      const AccT v = sSum[k];
-      if (v != AccT(0)) {
-        sSum[k] = AccT(0);
-        const uint32_t key = __umul24((uint32_t)k, 6554u) >> 16;   // k / 10 for k < 16384
-        const uint32_t id = __float_as_uint(sB[key].w);
-        AccT* row = (AccT*)accum + (uint64_t)id * 12;
-        if constexpr (kAccum == 0) atomicAdd(row + ((uint32_t)k - __umul24(key, 10u)), v);
-        else unsafeAtomicAdd(row + ((uint32_t)k - __umul24(key, 10u)), v);
+      for (int k = 10 * kPart * wv + lane; k < 10 * kPart * (wv + 1); k += 64) {
+        const uint32_t v = sSum[k];
+        if (v != 0u) {
+          sSum[k] = 0u;
+          const uint32_t key = __umul24((uint32_t)k, 6554u) >> 16;   // k / 10 for k < 16384
+          const uint32_t id = __float_as_uint(sB[key].w);
+          atomicAdd((uint32_t*)accum + (uint64_t)id * 12 + ((uint32_t)k - __umul24(key, 10u)), v);
+        }
       }
     }
+  };
+  // One visit, straight-line for all 64 lanes: the record at LDS offset jo
+  // from the three arrays' starts a0, b0 and c0; `before`: the key lies
+  // before this lane's end. Lanes that do not take the splat (outside the
+  // image, past their `end`, outside the cutoff, alpha below A_MIN, their
+  // group past its list) keep their state and contribute zero terms. Some
+  // lane took the splat in the forward, so there is nothing to vote on.
+  // add(w8): the previous visit's words to its sums; ready(): ahead of this
+  // visit's reduction. Returns the record's id.
+  const auto visit = [&](const float4* a0, const float4* b0, const float4* c0, uint32_t jo, bool before,
+                         auto&& add, auto&& ready) __attribute__((always_inline)) {
+    AccT w8[8];
+    red.read(w8);   // the previous visit's words
+    const float4 a = lds_at<float4>(a0, jo);
+    const float4 bb = lds_at<float4>(b0, jo);   // C, opa*comp, -0.5 cnorm, id
+    const float dx = px - a.x, dy = py - a.y;
+    const float cA = a.z, cB = a.w, cC = bb.x;
+    const float t2 = fmaf(cC * dy, dy, (cA * dx) * dx);
+    // clamped to [0, 87] as in the forward pass
+    const float e = clamp_e(fmaf(0.5f, t2, (cB * dx) * dy));
+    const float G = gs_expf_raster(-e);
+    const float araw = bb.y * G;
+    const float alpha = fminf(0.99f, araw);
+    const bool contrib = before && e <= cut.eCut && alpha >= cut.aMin;
+    const float4 c4 = lds_at<float4>(c0, jo);
+    // Tb = Ta / (1 - alpha), S / (1 - alpha) through one reciprocal.
+    // 1 - alpha lies in [0.0099, 1] (alpha in [0, 0.99]); on [2^-9, 1]
+    // v_rcp_f32 refined by one FMA Newton step equals the correctly
+    // rounded 1/x for every float (checked exhaustively on gfx950). A
+    // lane that does not take the splat has alpha 0 here: its reciprocal
+    // is exactly 1, so Tb = Ta and aT = 0 without a select each.
+    const float alphaE = contrib ? alpha : 0.0f;
+    const float rom = rcp_exact_unit(1.0f - alphaE);
+    const float Tb = Ta * rom;
+    add(w8);
+    const float gcol = fmaf(gCs[2], c4.z, fmaf(gCs[1], c4.y, gCs[0] * c4.x));   // scaled
+    // Every term is a product with galpha or aT, which are zero for the
+    // lanes that do not take the splat (all other factors are finite).
+    const float galphaS = (contrib && !(araw > 0.99f)) ? fmaf(gcol, Tb, -(GS * rom)) : 0.0f;
+    const float aT = alphaE * Tb;
+    const float ga = galphaS * araw;
+    const float gq = ga * bb.z;
+    const float gqdx = gq * dx;
+    float v[10];
+    v[0] = ga * (cA * dx + cB * dy);
+    v[1] = ga * (cB * dx + cC * dy);
+    v[2] = gqdx * dx;
+    v[3] = 2.0f * (gqdx * dy);        // the middle conic term is 2 gq dx dy
+    v[4] = (gq * dy) * dy;
+    v[5] = galphaS * c4.w * G;
+    v[6] = ga * (1.0f - c4.w);
+    v[7] = gCs[0] * aT;
+    v[8] = gCs[1] * aT;
+    v[9] = gCs[2] * aT;
+    GS = fmaf(gcol, aT, GS);
+    Ta = Tb;
+    AccT cur[10];
+    if constexpr (kAccum == 0) {
+      // i32(clamp(v * 16384, -1e9, 1e9)) per pixel; v already carries the
+      // scale. Terms beyond the clamp are rare, so one test of the largest
+      // magnitude stands for the clamps of the seven terms that carry
+      // galpha (they are NaN together, and then so is the maximum; a NaN
+      // converts to the lower clamp).
+      const float m = max3abs(max3abs(max3abs(v[0], v[1], v[2]), v[3], v[4]), v[5], v[6]);
+      if (wave_ballot(!(m <= 1.0e9f)) != 0ull) {
+#pragma unroll
+        for (int q = 0; q < 7; q++) v[q] = fminf(fmaxf(v[q], -1.0e9f), 1.0e9f);
+      }
+#pragma unroll
+      for (int q = 0; q < 10; q++)
+        cur[q] = (q >= 7 && kClampColour) ? (uint32_t)(int32_t)fminf(fmaxf(v[q], -1.0e9f), 1.0e9f)
+                                           : (uint32_t)(int32_t)v[q];
+    } else {
+#pragma unroll
+      for (int q = 0; q < 10; q++) cur[q] = v[q];
+    }
+    ready();
+    AccT h[5];
+    row_halve<AccT>(cur, h);
+    red.write(h);
+    return __float_as_uint(bb.w);
   };
   // batches start at multiples of 64 keys from s, so that their chunks are
   // the forward's chunks
@@ -659,127 +782,86 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
     }
     __syncthreads();
     const int pastEnd = (int)(myEnd - lo);   // this lane's end as an index of the batch
-    // each group's keys, last one first, then the record that nobody takes
-    constexpr uint32_t kNone = 0x01010101u * (uint32_t)kKeys;
-    int have[kGroups] = {};
-    for (int k = lane; k < kGroups * kKeys / 8; k += 64)
-      reinterpret_cast<uint2*>(sList + wv * kGroups * kKeys)[k] = make_uint2(kNone, kNone);
+    if constexpr (kAccum == 0) {
+      // each group's keys, last one first, then the record that nobody takes
+      constexpr uint32_t kNone = 0x01010101u * (uint32_t)kKeys;
+      int have[kGroups] = {};
+      for (int k = lane; k < kGroups * kKeys / 8; k += 64)
+        reinterpret_cast<uint2*>(sList + wv * kGroups * kKeys)[k] = make_uint2(kNone, kNone);
 #pragma unroll
-    for (int c = kKeys / 64 - 1; c >= 0; c--) {
+      for (int c = kKeys / 64 - 1; c >= 0; c--) {
 #pragma unroll
-      for (int q = 0; q < kGroups; q++) {
-        const uint32_t mLo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)words, kGroups * c + q);
-        const uint32_t mHi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(words >> 32), kGroups * c + q);
-        const uint64_t m = ((uint64_t)mHi << 32) | mLo;
-        const int cnt = __builtin_popcountll(m);
-        const uint32_t below = __builtin_amdgcn_mbcnt_hi(mHi, __builtin_amdgcn_mbcnt_lo(mLo, 0u));
-        if (__builtin_amdgcn_inverse_ballot_w64(m))
-          list[kKeys * (q - grp) + have[q] + cnt - 1 - (int)below] = (uint8_t)(64 * c + lane);
-        have[q] += cnt;
-      }
-    }
-    const int steps = max(max(have[0], have[1]), max(have[2], have[3]));
-    if (steps != 0) {
-      int nextKey = (int)list[0];
-      for (int step = 0; step < steps; step++) {
-        // Straight-line for all 64 lanes; lanes that do not take the splat
-        // (outside the image, past their `end`, outside the cutoff, alpha
-        // below A_MIN, their group past its list) keep their state and
-        // contribute zero terms. Some lane of the group took the splat in the
-        // forward, so there is nothing to vote on.
-        AccT w8[8];
-        red.read(w8);   // the previous visit's words
-        const int key = nextKey;
-        nextKey = (int)list[step + 1 < kKeys ? step + 1 : 0];
-        const uint32_t jo = (uint32_t)key * 16u;
-        const float4 a = lds_at<float4>(sA, jo);
-        const float4 bb = lds_at<float4>(sB, jo);   // C, opa*comp, -0.5 cnorm, id
-        const float dx = px - a.x, dy = py - a.y;
-        const float cA = a.z, cB = a.w, cC = bb.x;
-        const float t2 = fmaf(cC * dy, dy, (cA * dx) * dx);
-        // clamped to [0, 87] as in the forward pass
-        const float e = clamp_e(fmaf(0.5f, t2, (cB * dx) * dy));
-        const float G = gs_expf_raster(-e);
-        const float araw = bb.y * G;
-        const float alpha = fminf(0.99f, araw);
-        const bool contrib = key < pastEnd && e <= cut.eCut && alpha >= cut.aMin;
-        const float4 c4 = lds_at<float4>(sC, jo);
-        // Tb = Ta / (1 - alpha), S / (1 - alpha) through one reciprocal.
-        // 1 - alpha lies in [0.0099, 1] (alpha in [0, 0.99]); on [2^-9, 1]
-        // v_rcp_f32 refined by one FMA Newton step equals the correctly
-        // rounded 1/x for every float (checked exhaustively on gfx950). A
-        // lane that does not take the splat has alpha 0 here: its reciprocal
-        // is exactly 1, so Tb = Ta and aT = 0 without a select each.
-        const float alphaE = contrib ? alpha : 0.0f;
-        const float rom = rcp_exact_unit(1.0f - alphaE);
-        const float Tb = Ta * rom;
-        add_sum<kAccum>(sSum, lastKey, red.slot, red.total(w8), red.flusher);
-        const float gcol = fmaf(gCs[2], c4.z, fmaf(gCs[1], c4.y, gCs[0] * c4.x));   // scaled
-        // Every term is a product with galpha or aT, which are zero for the
-        // lanes that do not take the splat (all other factors are finite).
-        const float galphaS = (contrib && !(araw > 0.99f)) ? fmaf(gcol, Tb, -(GS * rom)) : 0.0f;
-        const float aT = alphaE * Tb;
-        const float ga = galphaS * araw;
-        const float gq = ga * bb.z;
-        const float gqdx = gq * dx;
-        float v[10];
-        v[0] = ga * (cA * dx + cB * dy);
-        v[1] = ga * (cB * dx + cC * dy);
-        v[2] = gqdx * dx;
-        v[3] = 2.0f * (gqdx * dy);        // the middle conic term is 2 gq dx dy
-        v[4] = (gq * dy) * dy;
-        v[5] = galphaS * c4.w * G;
-        v[6] = ga * (1.0f - c4.w);
-        v[7] = gCs[0] * aT;
-        v[8] = gCs[1] * aT;
-        v[9] = gCs[2] * aT;
-        GS = fmaf(gcol, aT, GS);
-        Ta = Tb;
-        AccT cur[10];
-        if constexpr (kAccum == 0) {
-          // i32(clamp(v * 16384, -1e9, 1e9)) per pixel; v already carries the
-          // scale. Terms beyond the clamp are rare, so one test of the largest
-          // magnitude stands for the clamps of the seven terms that carry
-          // galpha (they are NaN together, and then so is the maximum; a NaN
-          // converts to the lower clamp).
-          const float m = max3abs(max3abs(max3abs(v[0], v[1], v[2]), v[3], v[4]), v[5], v[6]);
-          if (wave_ballot(!(m <= 1.0e9f)) != 0ull) {
-#pragma unroll
-            for (int q = 0; q < 7; q++) v[q] = fminf(fmaxf(v[q], -1.0e9f), 1.0e9f);
-          }
-#pragma unroll
-          for (int q = 0; q < 10; q++)
-            cur[q] = (q >= 7 && kClampColour) ? (uint32_t)(int32_t)fminf(fmaxf(v[q], -1.0e9f), 1.0e9f)
-                                               : (uint32_t)(int32_t)v[q];
-        } else {
-#pragma unroll
-          for (int q = 0; q < 10; q++) cur[q] = v[q];
+        for (int q = 0; q < kGroups; q++) {
+          const uint32_t mLo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)words, kGroups * c + q);
+          const uint32_t mHi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(words >> 32), kGroups * c + q);
+          const uint64_t m = ((uint64_t)mHi << 32) | mLo;
+          const int cnt = __builtin_popcountll(m);
+          const uint32_t below = __builtin_amdgcn_mbcnt_hi(mHi, __builtin_amdgcn_mbcnt_lo(mLo, 0u));
+          if (__builtin_amdgcn_inverse_ballot_w64(m))
+            list[kKeys * (q - grp) + have[q] + cnt - 1 - (int)below] = (uint8_t)(64 * c + lane);
+          have[q] += cnt;
         }
-        // the next key has arrived by now: waited for here, not behind the
-        // writes below
-        asm volatile("" : "+v"(nextKey));
-        AccT h[5];
-        row_halve<AccT>(cur, h);
-        red.write(h);
-        lastKey = __builtin_amdgcn_ds_bpermute(keyFrom, key);
+      }
+      const int steps = max(max(have[0], have[1]), max(have[2], have[3]));
+      if (steps != 0) {
+        int nextKey = (int)list[0];
+        for (int step = 0; step < steps; step++) {
+          const int key = nextKey;
+          nextKey = (int)list[step + 1 < kKeys ? step + 1 : 0];
+          visit(sA, sB, sC, (uint32_t)key * 16u, key < pastEnd,
+                [&](const AccT* w8) { add_group_sums(sSum, lastKey, red.slot, red.total(w8), red.flusher); },
+                // the next key has arrived by now: waited for here, not behind the writes
+                [&]() { asm volatile("" : "+v"(nextKey)); });
+          lastKey = __builtin_amdgcn_ds_bpermute(keyFrom, key);
+        }
+      }
+      // the last visit's words, while its batch is staged
+      AccT w8[8];
+      red.read(w8);
+      add_group_sums(sSum, lastKey, red.slot, red.total(w8), red.flusher);
+      const AccT z[5] = {};
+      red.write(z);
+    } else {
+      // the keys that some group of the wave took, last one first
+#pragma unroll 1
+      for (int c = kKeys / 64 - 1; c >= 0; c--) {
+        uint32_t mLo = 0u, mHi = 0u;
+#pragma unroll
+        for (int q = 0; q < kGroups; q++) {
+          mLo |= (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)words, kGroups * c + q);
+          mHi |= (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(words >> 32), kGroups * c + q);
+        }
+        uint64_t m = ((uint64_t)mHi << 32) | mLo;
+        const int past = pastEnd - 64 * c;
+        while (m) {
+          const int bit = 63 - __builtin_clzll(m);
+          clear_bit(m, bit);
+          const uint32_t id =
+              visit(sA + 64 * c, sB + 64 * c, sC + 64 * c, lds_offset((uint32_t)bit * 16u), bit < past,
+                    [&](const AccT* w8) {
+                      add_wave_sums((float*)accum, lastId, red.slot, red.wave_total(w8), red.flusher && (lane & 3) == 0);
+                    },
+                    [] {});
+          lastId = id;
+        }
       }
     }
-    // the last visit's words, while its batch is staged
-    AccT w8[8];
-    red.read(w8);
-    add_sum<kAccum>(sSum, lastKey, red.slot, red.total(w8), red.flusher);
-    const AccT z[5] = {};
-    red.write(z);
     hi = lo;
   }
-  __syncthreads();
-  if (endMax > s) flush();
+  if constexpr (kAccum == 0) {
+    __syncthreads();
+    if (endMax > s) flush();
+  } else {
+    AccT w8[8];
+    red.read(w8);
+    add_wave_sums((float*)accum, lastId, red.slot, red.wave_total(w8), red.flusher && (lane & 3) == 0);
+  }
 }
 
 template <class S, int kLoss>
 __global__ __launch_bounds__(S::kThreads) void k_raster_fwd(Cam cam, Cut cut, RasterBufs b) {
   __shared__ float4 lds[RasterLds<S>::kFwd];
-  raster_fwd_tile<S, kLoss, kLoss == 2>(cam, cut, b, tile_of_block(b), lds);
+  raster_fwd_tile<S, kLoss, kLoss == 2 ? kTookGroups : kTookNone>(cam, cut, b, tile_of_block(b), lds);
 }
 
 template <class S, int kAccum, bool kClampColour>
@@ -798,7 +880,7 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::
   __shared__ float4 lds[RasterLds<S>::kBoth];   // the two passes' layouts share it
   const int tile = tile_of_block(b);
   PixelState ps;
-  raster_fwd_tile<S, 1, true>(cam, cut, b, tile, lds, &ps);
+  raster_fwd_tile<S, 1, kAccum == 0 ? kTookGroups : kTookWaves>(cam, cut, b, tile, lds, &ps);
   __syncthreads();   // the forward's last LDS reads are done
   raster_bwd_tile<S, kAccum, kClampColour>(cam, cut, b, accum, tile, lds, &ps);
 }
@@ -846,7 +928,7 @@ k_raster_fwd_bwd_views(const ViewBlock* __restrict__ vb, Cut cut, uint32_t* queu
     const Cam& cam = vb->cams[it.v];
     const RasterBufs& b = vb->bufs[it.v];
     PixelState ps;
-    raster_fwd_tile<S, 1, true>(cam, cut, b, it.tile, lds, &ps);
+    raster_fwd_tile<S, 1, kAccum == 0 ? kTookGroups : kTookWaves>(cam, cut, b, it.tile, lds, &ps);
     __syncthreads();   // the forward's last LDS reads are done
     raster_bwd_tile<S, kAccum, kClampColour>(cam, cut, b, gs_global(vb->accum[it.v]), it.tile, lds, &ps);
   }
@@ -862,7 +944,7 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(S::
   __shared__ float4 lds[RasterLds<S>::kBoth];
   const int tile = tile_of_block(b);
   PixelState ps;
-  raster_fwd_tile<S, 1, true>(cam, cut, b, tile, lds, &ps);
+  raster_fwd_tile<S, 1, kAccum == 0 ? kTookGroups : kTookWaves>(cam, cut, b, tile, lds, &ps);
   __syncthreads();
   raster_bwd_tile<S, kAccum, kClampColour>(cam, cut, b, gs_global(vb->accum[v]), tile, lds, &ps);
 }

@@ -726,6 +726,53 @@ def test_backward_lists_at_the_edges_of_their_batches(n, tile, batch):
     np.testing.assert_array_equal(out["data"].view(np.uint32), ref.P.view(np.uint32))
 
 
+@pytest.mark.parametrize("tile,batch", [(16, 256), (16, 64), (32, 256), (8, 128)])
+@pytest.mark.parametrize("n", [1, 63, 65, 128, 129, 257])
+@pytest.mark.parametrize("loss", ["charbonnier", "l1_dssim"])
+def test_f32_sums_at_the_edges_of_their_batches(n, tile, batch, loss):
+    """GS_ACCUM_F32 on the view above, both passes in one launch and in two:
+    every per-pixel term is the restatement's for the same dL/dC, only the
+    order of the sums differs. A sum of N f32 terms in
+    any order is within (N - 1) 2^-24 of the sum of their magnitudes (and the
+    terms' own sum in f64 is exact to 2^-53), here N = 384 pixels; the
+    magnitudes come from the restatement, one pixel at a time."""
+    print(n, tile, batch, loss, flush=True)
+    rng = np.random.default_rng(n)
+    W, H, f = 24, 16, 24.0
+    p = np.zeros((n, 16), np.float32)
+    z = rng.uniform(2.0, 4.0, n)
+    wide = rng.random(n) < 0.5
+    p[:, 0] = rng.uniform(-0.5, 0.5, n) * W / f * z
+    p[:, 1] = rng.uniform(-0.5, 0.5, n) * H / f * z
+    p[:, 2] = z
+    p[:, 3:6] = np.where(wide, np.log(1.0), np.log(0.02))[:, None] + rng.normal(0, 0.1, (n, 3))
+    p[:, 6] = 1.0
+    p[:, 10:13] = rng.normal(0, 1, (n, 3))
+    p[:, 13] = np.where(wide, -4.0, -1.0)
+    cams = [{"imgIdx": 0, "R": [1, 0, 0, 0, 1, 0, 0, 0, 1], "t": [0, 0, 0], "f": f, "cx": W / 2, "cy": H / 2, "w": W, "h": H}]
+    images = [{"tw": W, "th": H, "rgb": rng.random((H * W, 3)).astype(np.float32)}]
+    t = _trainer(p, None, cams, images, W, H, 1.0, {}, shDeg=0, tile=tile, batch=batch, gradAccum=gsabi.GS_ACCUM_F32,
+                 loss=gsabi.GS_LOSS_L1_DSSIM if loss == "l1_dssim" else gsabi.GS_LOSS_CHARBONNIER)
+    out = t.step_debug(0, want=("accum", "gC"))
+    t.destroy()
+    g = out["accum"].view(np.float32).astype(np.float64)
+    st = O.Stage(O.make_opts(shDeg=0), "f32")
+    cam = O.make_cam(cams[0], tile=tile)
+    proj, rect, cnt = st.project(cam, p, None)
+    ids, ts, _ = st.bin_sort(cam, proj, rect, cnt)
+    _, T, end = st.render_fwd(cam, proj, ids, ts)
+    gC = np.ascontiguousarray(out["gC"][:, :3])
+    valid = (out["gC"][:, 3] != 0).astype(np.uint8)
+    ref = st.render_bwd(cam, proj, ids, ts, T, end, gC, valid, fixed=False)
+    mag = np.zeros_like(ref)
+    for px in range(W * H):
+        one = np.zeros_like(valid)
+        one[px] = valid[px]
+        mag += np.abs(st.render_bwd(cam, proj, ids, ts, T, end, gC, one, fixed=False))
+    assert mag.any()
+    assert np.all(np.abs(g - ref) <= W * H * 2.0 ** -24 * mag + 1e-30)
+
+
 def test_psnr_reads_start_from_cleared_statistics():
     """A PSNR read leaves its statistics cleared for the next one; a training
     view rendered in between adds to them. The sums' atomics come in any

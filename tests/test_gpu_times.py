@@ -1,0 +1,61 @@
+"""One route of the trainer against another, timed side by side in one
+process: a launch that an option, a raster shape or a scene's size sends down
+its own path may not fall behind the path beside it. The limits leave room for
+noise; what they stand for is stated with each."""
+import numpy as np
+import pytest
+
+import gsabi
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(n, W, H, seed=0, ls=-4.0):
+    rng = np.random.default_rng(seed)
+    f = 0.6875 * W
+    p = np.zeros((n, 16), np.float32)
+    z = rng.uniform(3.0, 9.0, n)
+    p[:, 0] = rng.uniform(-0.6, 0.6, n) * W / f * z
+    p[:, 1] = rng.uniform(-0.6, 0.6, n) * H / f * z
+    p[:, 2] = z
+    p[:, 3:6] = ls + 0.3 * rng.normal(0, 1, (n, 3))
+    p[:, 6:10] = rng.normal(0, 1, (n, 4))
+    p[:, 6:10] /= np.linalg.norm(p[:, 6:10], axis=1, keepdims=True)
+    p[:, 10:13] = rng.normal(0, 1, (n, 3))
+    cams = [{"imgIdx": 0, "R": [1, 0, 0, 0, 1, 0, 0, 0, 1], "t": [0, 0, 0], "f": f, "cx": W / 2, "cy": H / 2, "w": W, "h": H}]
+    images = [{"tw": W, "th": H, "rgb": rng.random((W * H, 3)).astype(np.float32)}]
+    return p, cams, images
+
+
+def _stage_us(t, stage, steps=6, reps=5):
+    """The best of `reps` means of a stage's time over `steps` steps."""
+    for _ in range(4):
+        t.stepOnce(0)
+    best = float("inf")
+    for _ in range(reps):
+        t.profile(True)
+        for _ in range(steps):
+            t.stepOnce(0)
+        s = t.profile_read()[stage]
+        best = min(best, 1e3 * s["ms"] / s["launches"])
+        t.profile(False)
+    return best
+
+
+@pytest.mark.parametrize("tile", [8, 16, 32])
+def test_f32_sums_cost_no_more_than_fixed_point_ones(tile):
+    """GS_ACCUM_F32 adds the same terms as GS_ACCUM_FIXED, without their
+    conversion: its raster launch took 0.8-1.0 of the other's time before the
+    gradient sums of a batch moved to LDS, and up to 1.9 of it when float sums
+    went there too (LDS adds floats at a fraction of the rate of integers).
+    Limit 1.15."""
+    W, H = 1280, 720
+    p, cams, images = _scene(300000, W, H)
+    us = {}
+    for name, mode in (("fixed", gsabi.GS_ACCUM_FIXED), ("f32", gsabi.GS_ACCUM_F32)):
+        t = gsabi.GSTrainer(shDeg=0, maxSplats=p.shape[0], gradAccum=mode, tile=tile, posLr=1e-9)
+        t.setup({"data": p, "n": p.shape[0]}, cams, images, W, H, 2.0)
+        us[name] = _stage_us(t, "raster_fwd_bwd")
+        t.destroy()
+    print(tile, us, flush=True)
+    assert us["f32"] <= 1.15 * us["fixed"], us
