@@ -116,7 +116,7 @@ struct Shape {
 // LDS of the raster passes, carved from one array that the kernel declares,
 // so a launch that runs both passes holds the larger layout, not both.
 // Forward: records sA, sB, sC (16 B each per key), the chunk masks per
-// quadrant, the loss partials; backward: the records of a batch of 128 keys
+// quadrant, the loss partials; backward: the records of a batch of kKeys keys
 // and one that no lane takes, the waves' reduction scratch, the groups'
 // lists, the batch's gradient sums, the block's largest end. Sizes in float4.
 // 128 keys keep a block of 16-pixel tiles at 18.8 KB, eight to a CU.
@@ -124,7 +124,12 @@ constexpr int kRedStride = 68;   // words between a wave's 64-word rows (see Wav
 constexpr int kGroups = 4;       // 16-lane groups of a wave, each a 4x4 pixel block
 template <class S>
 struct RasterLds {
-  static constexpr int kKeys = S::B < 128 ? S::B : 128;   // keys per batch of the backward
+  // Keys per batch of the backward: 128, and 64 where the block is one wave
+  // (8-pixel tiles) and its forward stages no more than 128, since the CU then
+  // runs as many waves as its LDS holds blocks: 7.4 KB instead of 13.2. 1M
+  // Gaussians at 1920x1080, batches of 128: 1559 -> 1164 us (1505 when the
+  // backward held no lists and sums). With 256 the forward alone holds 12 KB.
+  static constexpr int kKeys = S::B < 128 || (S::T == 8 && S::B == 128) ? 64 : 128;
   static constexpr int kFwd = 3 * S::B + (S::kChunks * S::kMasks * 8 + 3 * S::kWaves * 8 + 15) / 16;
   static constexpr int kRed = S::kWaves * 5 * kRedStride / 4;   // the waves' reduction scratch
   static constexpr int kLists = S::kWaves * kGroups * kKeys / 16;   // a byte per key and group
