@@ -34,6 +34,7 @@
 // from device memory by every kernel; the grids are fixed. No pass uses
 // global atomics.
 #include "gs_kernels.h"
+#include "gs_bands.h"
 
 namespace gs {
 
@@ -1011,25 +1012,10 @@ struct ScatterPrep {
   }
 };
 
-// Tile rows per band of the scatter. Each of an XCD's blocks fills one line
-// of every tile's segment at a time; where those lines pass the XCD's 4 MB
-// L2, each 8-byte key goes to memory as a partial write of its own, and the
-// pass runs at that rate (77 Gkeys/s, as a bare kernel of such stores). So
-// the block takes the tiles in bands of rows whose open lines (128 bytes x
-// blocks per XCD x tiles) stay within 3 MB, and walks its Gaussians once per
-// band. 1920x1080, 1M Gaussians, 92.6M keys: 1156 us in one band, 694, 658
-// and 905 us in bands of 3, 6 and 12 rows (1.5, 2.9 and 5.9 MB).
-// A walk costs about 12 us however few keys it finds, so a segment run
-// shorter than a line does not pay: at 44, 26, 15, 9 and 5 keys per block and
-// tile the bands take 660, 433, 329, 259 and 217 us against 1156, 680, 405,
-// 249 and 162 without; the line is at 12.
-constexpr uint64_t kBandMinRun = 12;                     // keys per block and tile
-constexpr int kBandLines = (3 << 20) / 128;              // open lines per XCD
-
+// the scatter's bands of tile rows (gs_bands.h)
 __device__ __forceinline__ SegBands seg_bands(const SegJob& j) {
-  if (*j.totalKeys < kBandMinRun * (uint64_t)j.nb * (uint64_t)j.numTiles) return {1, 1};
-  const int tilesY = j.numTiles / j.tilesX, rows = kBandLines / ((j.nb + 7) / 8) / j.tilesX;
-  return {tilesY, rows < 1 ? 1 : rows < tilesY ? rows : tilesY};
+  const int tilesY = j.numTiles / j.tilesX;
+  return {tilesY, gs_band_rows(*j.totalKeys, j.n, j.nb, j.tilesX, tilesY)};
 }
 
 // Every (Gaussian, kept tile) key into its tile's segment: each tile's LDS
