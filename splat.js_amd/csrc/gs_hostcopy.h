@@ -2,11 +2,23 @@
 //
 // A copy to pageable memory runs at the rate at which one CPU thread copies
 // and, for a fresh array, faults its pages in: 13 GB/s for a 33 MB image.
-// Here the GPU fills the blocks of a small pinned ring and a few threads
+// Here kernels fill the blocks of a small pinned ring and a few threads
 // copy block after block to the caller while the next ones arrive. Renders
-// of 33 MB 3.0 -> 1.9 ms, reads of 73 MB of Gaussians 17 -> 2.5 ms (those
-// also pinned and freed their whole size on each call). 4, 8 and 12 threads,
-// and blocks of 1 and 2 MB, are within 10% of each other.
+// into fresh arrays against a plain copy: 64x64 132 -> 65 us, 480x360 290 ->
+// 211, 1280x720 1.16 -> 0.65 ms, 1920x1080 2.6 -> 1.3; a trainer's first one
+// 530 -> 230 us at 480x360, 1.25 -> 0.75 ms at 1280x720. Reads of 73 MB of
+// Gaussians 17.9 -> 2.4 ms (those also pinned and freed their whole size on
+// each call).
+//
+// Kernels, not the copy engine: a copy of its own behind a kernel starts up to
+// 130 us late. Through it the ring took 280 us for a 320x240 view that takes
+// 110-130 now (163-290 by a plain copy), and 430 instead of 210 at 480x360.
+// Four threads: their stacks stay in the C library's cache from call to call,
+// which keeps 40 MB (five of 8 MB). With six or eight a trainer's first render
+// took 1.1-2.4 ms at 1280x720 and 3.0-4.0 at 1920x1080 instead of 0.9 and 1.7;
+// later ones are within 5%. Blocks of 1 MB are within 10% of 2 MB, 0.5 MB cost
+// 20% more at 1920x1080. The first render of a program, 1920x1080: 14.9 ms by a
+// plain copy, 9.0 by the copy engine and eight threads, 3.1 now.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -26,7 +38,7 @@ namespace gs {
 struct HostRing {
   static constexpr int kSlots = 8;
   static constexpr size_t kSlotBytes = size_t(2) << 20;
-  static constexpr int kWorkers = 8;
+  static constexpr int kWorkers = 4;
   char* buf = nullptr;
   size_t have = 0;
   hipEvent_t ev[kSlots] = {};   // slot filled

@@ -326,6 +326,8 @@ struct RefineOp {
 // where clearSrc, and camWords words of camGrad.
 void launch_stats_read(hipStream_t st, double* src, double* window, double* out, bool clearSrc, uint32_t* camGrad,
                        int64_t camWords);
+// `count` pixels of img (RGBA floats) into out (pinned)
+void launch_pixels(hipStream_t st, int64_t count, const float4* img, float* out);
 // Rows [first, first + count) of the parameters (16 floats each) and of the SH
 // coefficients (C floats each; fmt 0 f32 planes, 1 bf16, 2 fp16) into out.
 void launch_param_rows(hipStream_t st, int64_t cap, int64_t first, int64_t count, const float4* P, float* out);

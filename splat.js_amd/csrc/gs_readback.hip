@@ -1,6 +1,7 @@
-// gs_readback.hip — what the host reads: the statistics of a loss or PSNR read,
-// and the Gaussians in the caller's layout (readGaussians, trainer.js:797-817): 16 floats and 3K coefficients per row, from the
-// 16-byte planes, written over PCIe straight into pinned host memory.
+// gs_readback.hip — what the host reads: a rendered view, the statistics of a
+// loss or PSNR read, and the Gaussians in the caller's layout (readGaussians,
+// trainer.js:797-817): 16 floats and 3K coefficients per row, from the 16-byte
+// planes. All are written over PCIe straight into pinned host memory.
 //
 // The device lays the rows out and decodes 16-bit coefficients, so that the
 // host only has to copy whole blocks: its loop over the planes took 7 of the
@@ -50,6 +51,17 @@ __global__ __launch_bounds__(1024) void k_stats_read(double* src, double* window
 void launch_stats_read(hipStream_t st, double* src, double* window, double* out, bool clearSrc, uint32_t* camGrad,
                        int64_t camWords) {
   k_stats_read<<<1, 1024, 0, st>>>(src, window, out, clearSrc, camGrad, camWords);
+}
+
+// pixels of a view as they are; PCIe bounds it
+__global__ __launch_bounds__(kBlock) void k_pixels(int64_t count, const float4* __restrict__ img, float4* __restrict__ out) {
+  const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (k < count) out[k] = img[k];
+}
+
+void launch_pixels(hipStream_t st, int64_t count, const float4* img, float* out) {
+  if (count <= 0) return;
+  k_pixels<<<(unsigned)((count + kBlock - 1) / kBlock), kBlock, 0, st>>>(count, img, (float4*)out);
 }
 
 void launch_param_rows(hipStream_t st, int64_t cap, int64_t first, int64_t count, const float4* P, float* out) {

@@ -1739,7 +1739,8 @@ int gs_render(gs_trainer_t* h, const gs_camera* c, int32_t trainMode, int64_t of
   const hipError_t e = ring_copy(
       h->ring, h->st, (int)((bytes + block - 1) / block), std::min(bytes, block),
       [&](int k, char* slot) {
-        return hipMemcpyAsync(slot, (const char*)h->img + k * block, size(k), hipMemcpyDeviceToHost, h->st);
+        launch_pixels(h->st, (int64_t)(size(k) / 16), h->img + k * (block / 16), (float*)slot);
+        return hipGetLastError();
       },
       [&](int k, const char* slot) { memcpy((char*)rgba + k * block, slot, size(k)); });
   if (e != hipSuccess) return hipfail(h, "renderView", e);
