@@ -74,13 +74,17 @@ struct HostRing {
 // `count` blocks of at most `bytes` (<= kSlotBytes) through the ring:
 // fill(k, slot) enqueues on st what writes block k into the pinned slot,
 // take(k, slot) copies it to the caller on any thread. Returns when all have
-// been taken, or with an error once nothing is being written or taken.
-template <typename Fill, typename Take>
-hipError_t ring_copy(HostRing& ring, hipStream_t st, int count, size_t bytes, Fill fill, Take take) {
+// been taken, or with an error once nothing is being written or taken. Where
+// the pinned memory cannot be had the call is plain(error)'s.
+template <typename Fill, typename Take, typename Plain>
+hipError_t ring_copy(HostRing& ring, hipStream_t st, int count, size_t bytes, Fill fill, Take take, Plain plain) {
   if (count <= 0) return hipSuccess;
   const size_t stride = std::min((bytes + 4095) / 4096 * 4096, HostRing::kSlotBytes);
   hipError_t e = ring.ensure(std::min(count, HostRing::kSlots), stride);
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return plain(e);
+  }
   const auto slot = [&](int k) { return ring.buf + (size_t)(k % HostRing::kSlots) * stride; };
   std::mutex m;
   std::condition_variable some, freed;

@@ -1742,7 +1742,11 @@ int gs_render(gs_trainer_t* h, const gs_camera* c, int32_t trainMode, int64_t of
         launch_pixels(h->st, (int64_t)(size(k) / 16), h->img + k * (block / 16), (float*)slot);
         return hipGetLastError();
       },
-      [&](int k, const char* slot) { memcpy((char*)rgba + k * block, slot, size(k)); });
+      [&](int k, const char* slot) { memcpy((char*)rgba + k * block, slot, size(k)); },
+      [&](hipError_t) {
+        const hipError_t c = hipMemcpyAsync(rgba, h->img, bytes, hipMemcpyDeviceToHost, h->st);
+        return c == hipSuccess ? hipStreamSynchronize(h->st) : c;
+      });
   if (e != hipSuccess) return hipfail(h, "renderView", e);
   return GS_OK;
 }
@@ -1840,7 +1844,8 @@ int gs_read_gaussians(gs_trainer_t* h, float* params, float* sh) {
         const bool p = k < kP;
         const int64_t rows = p ? rowsP : rowsS, width = p ? 16 : C, first = (p ? k : k - kP) * rows;
         memcpy((p ? params : sh) + first * width, slot, (size_t)(4 * width * std::min(rows, n - first)));
-      });
+      },
+      [](hipError_t err) { return err; });
   if (e != hipSuccess) return hipfail(h, "readGaussians", e);
   return GS_OK;
 }

@@ -12,7 +12,7 @@ typedef Stream* hipStream_t;
 typedef int* hipEvent_t;
 constexpr unsigned hipEventDisableTiming = 2, hipHostMallocDefault = 0;
 
-inline int pinned = 0, pinnedMost = 0, mallocsLeft = 1 << 30, eventsLeft = 1 << 30;
+inline int pinned = 0, pinnedMost = 0, mallocsLeft = 1 << 30, eventsLeft = 1 << 30, lastErrors = 0;
 
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   if (mallocsLeft-- <= 0) return hipErrorOutOfMemory;
@@ -48,3 +48,7 @@ inline hipError_t hipStreamSynchronize(hipStream_t s) {
   return hipSuccess;
 }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
+inline hipError_t hipGetLastError() {
+  lastErrors++;
+  return hipSuccess;
+}

@@ -22,6 +22,7 @@ using namespace gs;
 
 static std::mutex gm;
 static std::set<std::thread::id> takers;
+static hipError_t plain = hipSuccess;   // why the call was the caller's own
 
 // `count` blocks of `bytes`: block k holds bytes (k + i) & 0xff; failAt: that fill fails
 static int copy(HostRing& ring, int count, size_t bytes, int failAt, hipError_t* err) {
@@ -29,6 +30,7 @@ static int copy(HostRing& ring, int count, size_t bytes, int failAt, hipError_t*
   Stream st;
   std::atomic<int> taken{0};
   takers.clear();
+  plain = hipSuccess;
   *err = ring_copy(
       ring, &st, count, bytes,
       [&](int k, char* slot) {
@@ -40,7 +42,12 @@ static int copy(HostRing& ring, int count, size_t bytes, int failAt, hipError_t*
         { std::lock_guard<std::mutex> l(gm); takers.insert(std::this_thread::get_id()); }
         taken++;
         memcpy(out.data() + (size_t)k * bytes, slot, bytes);
+      },
+      [&](hipError_t why) {   // the caller's own copy
+        plain = why;
+        return hipSuccess;
       });
+  if (plain != hipSuccess) return 0;
   if (*err != hipSuccess) return st.syncs == 1 && taken <= failAt ? 0 : 1;
   for (int k = 0; k < count; k++)
     for (size_t i = 0; i < bytes; i++)
@@ -50,19 +57,19 @@ static int copy(HostRing& ring, int count, size_t bytes, int failAt, hipError_t*
 
 int main(int argc, char** argv) {
   const std::string mode = argv[1];
-  if (mode == "nomem") {   // pinned memory or an event that cannot be had: the error, and nothing left half made
+  if (mode == "nomem") {   // pinned memory or an event that cannot be had: the caller's copy, no error left behind
     HostRing r;
     hipError_t e;
     int bad = 0;
     mallocsLeft = 0;
     copy(r, 4, 1000, 0, &e);
-    bad |= e != hipErrorOutOfMemory || r.have != 0 || r.buf != nullptr;
+    bad |= e != hipSuccess || plain != hipErrorOutOfMemory || lastErrors != 1 || r.have != 0 || r.buf != nullptr;
     mallocsLeft = 1 << 30;
     eventsLeft = 2;
     copy(r, 4, 1000, 0, &e);
-    bad |= e != hipErrorUnknown;
+    bad |= e != hipSuccess || plain != hipErrorUnknown || lastErrors != 2;
     eventsLeft = 1 << 30;
-    bad |= copy(r, 4, 1000, -1, &e) || e != hipSuccess;
+    bad |= copy(r, 4, 1000, -1, &e) || e != hipSuccess || plain != hipSuccess;
     r.release();
     printf("%d %d\n", bad, pinned);
     return 0;
