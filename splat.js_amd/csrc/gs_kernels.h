@@ -243,9 +243,9 @@ struct RasterShape {
   int tile, batch;
 };
 bool raster_shape_ok(int tile, int batch);
-// bytes of RasterBufs::took for views of up to w x h pixels and `keys` sorted
-// keys, enough at every raster shape
-size_t raster_took_bytes(int w, int h, int64_t keys);
+// bytes of RasterBufs::took for a w x h view in tiles of `tile` pixels with
+// `keys` sorted keys
+size_t raster_took_bytes(int tile, int w, int h, int64_t keys);
 
 // loss: 0 none (view render), 1 Charbonnier fused into the forward pass,
 // 2 forward only, loss computed by a separate kernel

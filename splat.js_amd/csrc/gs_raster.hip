@@ -969,15 +969,10 @@ static void with_shape(const RasterShape& sh, F&& f) {
   else with_batch<16>(sh.batch, f);
 }
 
-size_t raster_took_bytes(int w, int h, int64_t keys) {
-  // took_word's last row at each tile size: one word per 4x4 pixels
-  size_t words = 0;
-  for (int t = 8; t <= 32; t *= 2) {
-    const size_t tiles = (size_t)((w + t - 1) / t) * (size_t)((h + t - 1) / t);
-    const size_t need = ((size_t)keys / 64 + tiles + 1) * (size_t)(t * t / 16);
-    words = words > need ? words : need;
-  }
-  return words * 8;
+size_t raster_took_bytes(int tile, int w, int h, int64_t keys) {
+  // rows of one word per 4x4 pixels, up to took_word's last
+  const size_t tiles = (size_t)((w + tile - 1) / tile) * (size_t)((h + tile - 1) / tile);
+  return ((size_t)keys / 64 + tiles + 1) * (size_t)(tile * tile / 16) * 8;
 }
 
 bool raster_shape_ok(int tile, int batch) {

@@ -94,6 +94,8 @@ struct gs_trainer {
   int maxTiles = 0;      // tiles of the largest view at the smallest tile size (8): every shape fits
   int64_t maxPix = 0;
   RasterShape shape{kDefaultTile, kDefaultBatch};   // raster tile side and LDS batch
+  std::vector<uint64_t*> tookOwn;   // RasterBufs::took of the slots that have no sort buffers to lend (else null)
+  size_t tookOwnBytes = 0;          // each of them: enough at the current tile size
 
   HostRing ring;                        // pinned blocks of the large synchronous reads
   std::shared_ptr<StatPool> statPool;   // pinned blocks of the loss and PSNR reads
@@ -119,7 +121,6 @@ struct gs_trainer {
   float* Tfin = nullptr;
   uint32_t* endIdx = nullptr;
   float4* gC = nullptr;
-  uint64_t* took = nullptr;      // the training forward's taken keys (RasterBufs::took)
   float* ssimScratch = nullptr;  // 9 x maxPix SSIM partials (L1 + D-SSIM loss only)
   uint32_t* targets = nullptr;
   int64_t totalPx = 0;
@@ -154,7 +155,7 @@ struct gs_trainer {
   // buffers; slot 0 is the single-view set above
   struct ViewSlot {
     float4* rec; uint32_t* cnt; void* accum; uint32_t* ids; uint2* ranges; uint32_t* tileOrder;
-    float4* img; float* T; uint32_t* end; float4* gC; uint64_t* took;
+    float4* img; float* T; uint32_t* end; float4* gC;
     // the batched binning's own copies (slot 0: the single-view buffers)
     uint32_t* depthKey; uint2* rect; uint32_t* chunkKeys; uint32_t* blockStart; uint32_t* table;
     uint32_t* visPart; uint32_t* tileCnt; uint64_t* keys; uint64_t* tmp; uint64_t* totalKeys;
@@ -269,6 +270,10 @@ void free_all(gs_trainer* h) {
   }
   for (void* p : h->allocs) (void)hipFree(p);
   h->allocs.clear();
+  for (uint64_t* p : h->tookOwn)
+    if (p) (void)hipFree(p);
+  h->tookOwn.clear();
+  h->tookOwnBytes = 0;
   h->vslots.clear();
   h->ready = false;
 }
@@ -468,6 +473,49 @@ void radix_values_into(BinArgs& a, uint32_t* ids, uint32_t* scratch) {
   a.tvB = passes % 2 ? ids : scratch;
 }
 
+// ---- where the training raster's taken keys go (RasterBufs::took) ----
+// They take up to 8 bytes per key of the budget (32-pixel tiles; 2 at 16), so
+// they lie in sort buffers that are free once a view is binned, whose sizes
+// allow for them:
+// - slot 0 and single views: the key and id buffers that the sorted ids are
+//   not in (keys and ids are allocated in two such pairs);
+// - further slots with batched binning: their segment keys.
+// Two cases have none and get a buffer of their own, for the tile size in use:
+// slot 0 of the overlapped launches, whose raster runs beside the next view's
+// binning through the shared buffers, and slots without binning buffers.
+uint64_t* single_took(const gs_trainer* h) {
+  return (uint64_t*)(h->lastBin.ids == h->tvB ? h->tkA : h->tkB);
+}
+bool took_is_own(const gs_trainer* h, size_t slot) {
+  return slot == 0 ? h->o.viewsLaunch == GS_VIEWS_OVERLAP : !h->batchedBin;
+}
+uint64_t* view_took(const gs_trainer* h, size_t slot) {
+  if (took_is_own(h, slot)) return h->tookOwn[slot];
+  return slot == 0 ? (uint64_t*)h->tkB : h->vslots[slot].keys;
+}
+
+// The buffers of their own, large enough for tiles of `tile` pixels. Where that
+// fails the trainer keeps those it has.
+int fit_took(gs_trainer* h, int tile) {
+  if (h->vslots.size() < 2 || h->o.sortMode != GS_SORT_TILE_SEGMENTS) return GS_OK;   // no batched steps
+  size_t need = 0;
+  for (const CamMeta& m : h->cams) need = std::max(need, raster_took_bytes(tile, m.c.w, m.c.h, h->entriesCap));
+  if (need <= h->tookOwnBytes) return GS_OK;
+  std::vector<uint64_t*> own(h->vslots.size(), nullptr);
+  hipError_t e = hipSuccess;
+  for (size_t k = 0; k < own.size() && e == hipSuccess; k++)
+    if (took_is_own(h, k)) e = hipMalloc((void**)&own[k], need);
+  if (e == hipSuccess) own.swap(h->tookOwn);
+  for (uint64_t* p : own)
+    if (p) (void)hipFree(p);   // waits for the device
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(h, GS_E_NOMEM, "hipMalloc(" + std::to_string(need) + " B) failed: " + hipGetErrorString(e));
+  }
+  h->tookOwnBytes = need;
+  return GS_OK;
+}
+
 // ---- one raster: project -> bin/sort -> forward (+ loss) ----
 int run_raster(gs_trainer* h, const Cam& cam, int loss, double* statsBuf, bool withBwd = false) {
   const int64_t n = h->n;
@@ -522,7 +570,7 @@ int run_raster(gs_trainer* h, const Cam& cam, int loss, double* statsBuf, bool w
   b.T = h->Tfin;
   b.end = h->endIdx;
   b.gC = h->gC;
-  b.took = h->took;
+  b.took = single_took(h);
   b.tgt = h->targets;
   b.stats = statsBuf;
   if (withBwd) {
@@ -757,7 +805,7 @@ int step_impl(gs_trainer* h, int ci, gs_debug_out* dbg) {
   b.T = h->Tfin;
   b.end = h->endIdx;
   b.gC = h->gC;
-  b.took = h->took;
+  b.took = single_took(h);
   if (ssim) {
     Scope s(h, "raster_bwd", 0.0);
     launch_raster_bwd(h->st, h->shape, cam, make_cut(h), b, h->o.gradAccum, h->accum, false);
@@ -1019,7 +1067,7 @@ int fill_views(gs_trainer* h, const int* ci, int count, int activeDeg, double* s
     b.T = sl.T;
     b.end = sl.end;
     b.gC = sl.gC;
-    b.took = sl.took;
+    b.took = view_took(h, (size_t)k);
     b.tgt = h->targets;
     b.stats = statsBuf;
     vb.accum[k] = sl.accum;
@@ -1364,10 +1412,17 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
   rc |= dalloc(h, &h->dkB, (size_t)cap * 4);
   rc |= dalloc(h, &h->dvB, (size_t)cap * 4);
   const size_t kb = h->o.sortMode == GS_SORT_DEPTH_THEN_TILE ? 4 : 8;
-  rc |= dalloc(h, &h->tkA, (size_t)h->entriesCap * kb);
-  rc |= dalloc(h, &h->tkB, (size_t)h->entriesCap * kb);
-  rc |= dalloc(h, &h->tvA, (size_t)h->entriesCap * 4);
-  rc |= dalloc(h, &h->tvB, (size_t)h->entriesCap * 4);
+  // keys and ids in two pairs; the pair that the sorted ids are not in also
+  // holds the raster's taken keys (single_took)
+  size_t tookBytes = 0;
+  for (const CamMeta& m : h->cams)
+    for (int t = 8; t <= 32; t *= 2) tookBytes = std::max(tookBytes, raster_took_bytes(t, m.c.w, m.c.h, h->entriesCap));
+  const size_t keysAt = ((size_t)h->entriesCap * kb + 255) / 256 * 256;
+  const size_t pair = std::max(keysAt + (size_t)h->entriesCap * 4, tookBytes);
+  rc |= dalloc(h, &h->tkA, pair);
+  rc |= dalloc(h, &h->tkB, pair);
+  h->tvA = (uint32_t*)((char*)h->tkA + keysAt);
+  h->tvB = (uint32_t*)((char*)h->tkB + keysAt);
   h->sort.G = kSortBlocks;
   rc |= dalloc(h, &h->sort.hist, (size_t)256 * kSortBlocks * 4);
   rc |= dalloc(h, &h->sort.totals, 256 * 4);
@@ -1400,9 +1455,6 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
   rc |= dalloc(h, &h->Tfin, (size_t)h->maxPix * 4);
   rc |= dalloc(h, &h->endIdx, (size_t)h->maxPix * 4);
   rc |= dalloc(h, &h->gC, (size_t)h->maxPix * 16);
-  size_t tookBytes = 0;
-  for (const CamMeta& m : h->cams) tookBytes = std::max(tookBytes, raster_took_bytes(m.c.w, m.c.h, h->entriesCap));
-  rc |= dalloc(h, &h->took, tookBytes);
   if (h->o.loss == GS_LOSS_L1_DSSIM) rc |= dalloc(h, &h->ssimScratch, (size_t)h->maxPix * 36);
   rc |= dalloc(h, &h->targets, tgt.size() * 4);
   rc |= dalloc(h, &h->stats, 8 * kStatDoubles);
@@ -1411,7 +1463,7 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
   // batched views: slot 0 is the single-view set, slots 1.. their own copies
   h->vslots.assign((size_t)h->o.viewsPerStep, gs_trainer::ViewSlot{});
   h->vslots[0] = {h->rec, h->cnt, h->accum, h->tvA, h->ranges, h->tileOrder, h->img, h->Tfin, h->endIdx, h->gC,
-                  h->took, h->depthKey, h->rect, h->sort.chunkKeys, h->sort.blockStart, h->sort.segTable, h->sort.visPart,
+                  h->depthKey, h->rect, h->sort.chunkKeys, h->sort.blockStart, h->sort.segTable, h->sort.visPart,
                   h->sort.tileCnt, (uint64_t*)h->tkA, (uint64_t*)h->tkB, h->totalKeys};
   for (size_t k = 1; k < h->vslots.size(); k++) {
     gs_trainer::ViewSlot& v = h->vslots[k];
@@ -1425,7 +1477,6 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
     rc |= dalloc(h, &v.T, (size_t)h->maxPix * 4);
     rc |= dalloc(h, &v.end, (size_t)h->maxPix * 4);
     rc |= dalloc(h, &v.gC, (size_t)h->maxPix * 16);
-    rc |= dalloc(h, &v.took, tookBytes);
   }
   if (h->o.viewsPerStep > 1) {
     rc |= dalloc(h, &h->dVB, sizeof(ViewBlock));
@@ -1452,7 +1503,7 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
         rc |= dalloc(h, &v.table, (size_t)rows * segTiles * 4);
         rc |= dalloc(h, &v.visPart, (size_t)rows * 4);
         rc |= dalloc(h, &v.tileCnt, (size_t)h->maxTiles * 4);
-        rc |= dalloc(h, &v.keys, (size_t)h->entriesCap * 8);
+        rc |= dalloc(h, &v.keys, std::max((size_t)h->entriesCap * 8, tookBytes));   // and the taken keys (view_took)
         rc |= dalloc(h, &v.tmp, (size_t)h->entriesCap * 8);
         rc |= dalloc(h, &v.totalKeys, 8);
         // the projection adds to these sums and the scan clears them after use
@@ -1461,6 +1512,7 @@ int gs_setup(gs_trainer_t* h, const float* params, int64_t n, const float* sh, c
       h->batchedBin = rc == 0;
     }
   }
+  if (rc == 0) rc = fit_took(h, h->shape.tile);
   if (rc) { free_all(h); return rc < 0 ? rc : GS_E_NOMEM; }
   if (h->o.viewsPerStep > 1) {
     hipError_t e = hipHostMalloc((void**)&h->hVB, sizeof(ViewBlock) * kRing, hipHostMallocDefault);
@@ -1544,10 +1596,13 @@ int gs_step_views_debug(gs_trainer_t* h, const int32_t* cams, int32_t count, gs_
 
 namespace {
 
-void set_shape(gs_trainer* h, const RasterShape& sh) {
-  if (sh.tile == h->shape.tile && sh.batch == h->shape.batch) return;
+int set_shape(gs_trainer* h, const RasterShape& sh) {
+  if (sh.tile == h->shape.tile && sh.batch == h->shape.batch) return GS_OK;
+  const int rc = h->ready ? fit_took(h, sh.tile) : GS_OK;
+  if (rc) return rc;
   h->shape = sh;
   if (h->dVB) h->viewBlocks = raster_views_blocks(h->o.device, sh);
+  return GS_OK;
 }
 
 // One autotuning pass over cameras ci[0..count) at the current shape: the
@@ -1579,7 +1634,7 @@ int tune_pass(gs_trainer* h, const int* ci, int count, int activeDeg) {
     b.T = h->Tfin;
     b.end = h->endIdx;
     b.gC = h->gC;
-    b.took = h->took;
+    b.took = single_took(h);
     launch_raster_bwd(h->st, h->shape, cam, make_cut(h), b, h->o.gradAccum, h->accum, false);
     HIPCK(hipGetLastError());
     return GS_OK;
@@ -1604,8 +1659,7 @@ int gs_set_raster_shape(gs_trainer_t* h, int32_t tile, int32_t batch) {
   if (!raster_shape_ok(tile, batch))
     return fail(h, GS_E_ARG, "raster shape: tile 8, 16 or 32 and batch 64, 128 or 256");
   HIPCK(hipSetDevice(h->o.device));
-  set_shape(h, RasterShape{tile, batch});
-  return GS_OK;
+  return set_shape(h, RasterShape{tile, batch});
 }
 
 int gs_autotune(gs_trainer_t* h, const int32_t* cams, int32_t count, int32_t reps, gs_tune_entry* out) {
@@ -1639,7 +1693,8 @@ int gs_autotune(gs_trainer_t* h, const int32_t* cams, int32_t count, int32_t rep
   }
   for (int i = 0; i < 9 && rc == GS_OK; i++) {
     gs_tune_entry& en = out[i];
-    set_shape(h, RasterShape{en.tile, en.batch});
+    rc = set_shape(h, RasterShape{en.tile, en.batch});
+    if (rc) break;
     // warm-up pass: also gives the pass's keys and budget drops
     if (hipMemsetAsync(h->evalStats, 0, 8 * kStatDoubles, h->st) != hipSuccess) { rc = hipfail(h, "autotune", hipGetLastError()); break; }
     rc = tune_pass(h, ci, count, activeDeg);
@@ -1670,7 +1725,7 @@ int gs_autotune(gs_trainer_t* h, const int32_t* cams, int32_t count, int32_t rep
   launch_fill_u32(h->st, (uint32_t*)h->evalStats, 2 * kStatDoubles, 0u);
   HIPCK(hipStreamSynchronize(h->st));
   if (rc) {
-    set_shape(h, start);
+    (void)set_shape(h, start);
     return rc;
   }
   // eligible: measured, and dropping no more keys than the reference's 16-pixel tiles
@@ -1684,8 +1739,7 @@ int gs_autotune(gs_trainer_t* h, const int32_t* cams, int32_t count, int32_t rep
     }
     if (best < 0 || out[i].ms < out[best].ms) best = i;
   }
-  set_shape(h, best >= 0 ? RasterShape{out[best].tile, out[best].batch} : start);
-  return GS_OK;
+  return set_shape(h, best >= 0 ? RasterShape{out[best].tile, out[best].batch} : start);
 }
 
 int gs_step_batch(gs_trainer_t* h, const int32_t* cams, int32_t count) {
