@@ -274,6 +274,7 @@ void free_all(gs_trainer* h) {
     if (p) (void)hipFree(p);
   h->tookOwn.clear();
   h->tookOwnBytes = 0;
+  h->batchedBin = false;
   h->vslots.clear();
   h->ready = false;
 }

@@ -18,9 +18,8 @@ def _free_bytes():
     return free.value
 
 
-def _setup(keys, W=160, H=96, **kw):
+def _setup(keys, W=160, H=96, n=500, trainer=None, **kw):
     rng = np.random.default_rng(1)
-    n = 500
     p = np.zeros((n, 16), np.float32)
     z = rng.uniform(2.0, 4.0, n)
     p[:, 0] = rng.uniform(-0.5, 0.5, n) * W / 100.0 * z
@@ -30,7 +29,7 @@ def _setup(keys, W=160, H=96, **kw):
     p[:, 6] = 1.0
     cams = [{"imgIdx": 0, "R": [1, 0, 0, 0, 1, 0, 0, 0, 1], "t": [0, 0, 0], "f": 100.0, "cx": W / 2, "cy": H / 2, "w": W, "h": H}]
     images = [{"tw": W, "th": H, "rgb": rng.random((W * H, 3)).astype(np.float32)}]
-    t = gsabi.GSTrainer(shDeg=0, maxSplats=n, entriesCap=keys, **kw)
+    t = trainer or gsabi.GSTrainer(shDeg=0, maxSplats=n, entriesCap=keys, **kw)
     t.setup({"data": p, "n": n}, cams, images, W, H, 2.0)
     return t
 
@@ -82,3 +81,23 @@ def test_raster_shapes_changed_between_batched_steps(launch):
         np.testing.assert_array_equal(x.view(np.uint32), y.view(np.uint32), err_msg=f"tile {tile}")
     a.destroy()
     b.destroy()
+
+
+def test_second_setup_past_the_batched_binning_limit():
+    """15 further slots of 107.3M keys take 25.76 GB of binning buffers, just
+    under the 24 GiB that batched binning may have; with 100k Gaussians the
+    same trainer's second setup passes that, and its views bin one after
+    another. Its steps are those of a trainer that was set up once."""
+    kw = dict(viewsPerStep=16, seed=5)
+    keys = 107_300_000
+    a = _setup(keys, n=500, **kw)
+    a.stepViews([0, 0])
+    _setup(keys, n=100000, trainer=a)
+    b = _setup(1 << 22, n=100000, **kw)
+    for t in (a, b):
+        for _ in range(3):
+            t.stepViews([0, 0, 0])
+    x, y = a.readGaussians()["data"], b.readGaussians()["data"]
+    a.destroy()
+    b.destroy()
+    np.testing.assert_array_equal(x.view(np.uint32), y.view(np.uint32))
