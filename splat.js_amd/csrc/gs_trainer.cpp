@@ -1883,6 +1883,7 @@ int gs_read_gaussians(gs_trainer_t* h, float* params, float* sh) {
   const int64_t n = h->n, C = sh ? h->shC : 0;
   const int64_t rowsP = (int64_t)(HostRing::kSlotBytes / 64), rowsS = C ? (int64_t)(HostRing::kSlotBytes / (4 * C)) : 1;
   const int kP = params ? (int)((n + rowsP - 1) / rowsP) : 0, kS = C ? (int)((n + rowsS - 1) / rowsS) : 0;
+  if (kP + kS == 0) HIPCK(hipStreamSynchronize(h->st));   // nothing to read: waits, as a read does
   const size_t most = 4 * (size_t)std::max(kP ? 16 * std::min(rowsP, n) : 0, kS ? C * std::min(rowsS, n) : 0);
   const hipError_t e = ring_copy(
       h->ring, h->st, kP + kS, most,

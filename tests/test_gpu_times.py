@@ -79,3 +79,27 @@ def test_batches_of_8_pixel_tiles_cost_alike():
     t.destroy()
     print(ms, flush=True)
     assert ms[128] <= 1.08 * ms[64], ms
+
+
+def test_a_read_of_nothing_waits_as_any_read():
+    """gs_read_gaussians with neither array waits for the enqueued steps (some
+    20 ms of them here): a sync behind it finds nothing left to wait for."""
+    import time
+    W, H = 1280, 720
+    p, cams, images = _scene(300000, W, H)
+    t = gsabi.GSTrainer(shDeg=0, maxSplats=p.shape[0], posLr=1e-9)
+    t.setup({"data": p, "n": p.shape[0]}, cams, images, W, H, 2.0)
+    for _ in range(5):
+        t.stepOnce(0)
+    t.sync()
+    a = time.perf_counter()
+    for _ in range(40):
+        t.stepOnce(0)
+    b = time.perf_counter()
+    assert gsabi.lib().gs_read_gaussians(t._h, None, None) == 0
+    c = time.perf_counter()
+    t.sync()
+    d = time.perf_counter()
+    t.destroy()
+    print("enqueue %.2f read %.2f sync %.2f ms" % (1e3 * (b - a), 1e3 * (c - b), 1e3 * (d - c)), flush=True)
+    assert c - a > 5e-3 and d - c < 2e-3
