@@ -513,6 +513,80 @@ def test_entry_budget_drops_whole_tiles_as_the_reference():
     t.destroy()
 
 
+def _budget_scene(n, W, H, wide, seed=3):
+    """n splats over a W x H view, a third of them in its middle (segments past
+    2048 keys), the first `wide` of them over all of it."""
+    rng = np.random.default_rng(seed)
+    f = float(W)
+    p = np.zeros((n, 16), np.float32)
+    z = rng.uniform(2.0, 4.0, n)
+    spread = np.where(np.arange(n) % 3 == 0, 0.04, 1.0)
+    p[:, 0] = rng.uniform(-0.5, 0.5, n) * spread * W / f * z
+    p[:, 1] = rng.uniform(-0.5, 0.5, n) * spread * H / f * z
+    p[:, 2] = z
+    p[:, 3:6] = np.log(0.03) + rng.normal(0, 0.1, (n, 3))
+    p[:wide, 0:2] = 0.0
+    p[:wide, 3:6] = np.log(4.0)
+    p[:, 6] = 1.0
+    p[:, 10:13] = rng.normal(0, 1, (n, 3))
+    p[:, 13] = rng.uniform(-4, -1, n)
+    cams = [{"imgIdx": 0, "R": [1, 0, 0, 0, 1, 0, 0, 0, 1], "t": [0, 0, 0], "f": f, "cx": W / 2, "cy": H / 2, "w": W, "h": H}]
+    images = [{"tw": W, "th": H, "rgb": np.full((W * H, 3), 0.5, np.float32)}]
+    return p, cams, images
+
+
+@pytest.mark.parametrize("share", [0.05, 0.6, 0.98])
+@pytest.mark.parametrize("W,H,n,wide", [(690, 395, 20000, 0), (955, 555, 20000, 0), (1195, 890, 30000, 0), (1995, 1147, 30000, 0),
+                                        (640, 480, 300000, 3000)],
+                         ids=["1100_tiles", "2100_tiles", "4200_tiles", "9000_tiles", "bands"])
+def test_entry_budget_at_every_width_of_the_scan(W, H, n, wide, share):
+    """The budget's end inside a chunk of 64 tiles, for each number of tiles
+    that a thread of the scan takes (2, 4, 8 and 16; 1 in the test above), most
+    tiles dropped, about half, and fewer; the last chunks are not full. In the
+    last view the scatter also takes the tiles in bands of rows. The
+    kept keys, ranges and dropped tiles are the restatement's budget applied to
+    the radix strategy's keys."""
+    p, cams, images = _budget_scene(n, W, H, wide)
+    kw = dict(shDeg=0, radClamp=2000.0)
+    t = _trainer(p, None, cams, images, W, H, 1.0, {}, sortMode=gsabi.GS_SORT_DEPTH_THEN_TILE, entriesCap=1 << 24, **kw)
+    r = t.step_debug(0, want=("ids", "keys", "tileRanges"))
+    t.destroy()
+    tiles = -(-W // 16) * -(-H // 16)
+    ts = np.searchsorted(r["keys"] >> np.uint64(32), np.arange(tiles + 1, dtype=np.uint64)).astype(np.uint32)
+    cap = int(share * r["numKeys"])
+    ids, keys, ts2, dropped = O.apply_tile_budget(r["ids"], r["keys"], ts, cap)
+    assert 0 < dropped < tiles and 0 < len(ids) < r["numKeys"]
+    if wide:   # keys for bands: 12 per block and tile
+        assert r["numKeys"] >= 12 * 256 * tiles
+    t = _trainer(p, None, cams, images, W, H, 1.0, {}, entriesCap=cap, **kw)
+    g = t.step_debug(0, want=("ids", "keys", "tileRanges"))
+    stats = t.step_stats()
+    t.destroy()
+    assert g["numKeys"] == stats.lastKeys == len(ids) and stats.overflowKeys == dropped
+    np.testing.assert_array_equal(g["ids"], ids)
+    np.testing.assert_array_equal(g["keys"], keys)
+    tr = g["tileRanges"].astype(np.int64)
+    np.testing.assert_array_equal(tr[:, 0], ts2[:-1])
+    np.testing.assert_array_equal(tr[:, 1], ts2[1:])
+
+
+def test_rounds_full_of_wide_splats_as_the_radix_strategy():
+    """270,000 splats over all 100 tiles of a view: every block's round of 1024
+    Gaussians holds 102,400 keys, walked in two windows of 65536. (The budget
+    counts 2^19 keys for each tile's 270,000.)"""
+    p, cams, images = _budget_scene(270000, 160, 160, 270000)
+    outs = []
+    for mode in (gsabi.GS_SORT_TILE_SEGMENTS, gsabi.GS_SORT_DEPTH_THEN_TILE):
+        t = _trainer(p, None, cams, images, 160, 160, 1.0, {}, shDeg=0, sortMode=mode, radClamp=2000.0, entriesCap=1 << 26)
+        outs.append(t.step_debug(0, want=("ids", "keys", "tileRanges")))
+        t.destroy()
+    a, b = outs
+    assert a["numKeys"] == b["numKeys"] == 270000 * 100
+    np.testing.assert_array_equal(a["keys"], b["keys"])
+    np.testing.assert_array_equal(a["ids"], b["ids"])
+    np.testing.assert_array_equal(a["tileRanges"], b["tileRanges"])
+
+
 def test_radix_sort_budget_drops_keys_in_sort_order():
     """The radix strategies keep the first `entriesCap` keys of the sorted
     order instead."""
