@@ -109,7 +109,7 @@ struct SegJob {
   uint64_t* totalKeys;
   double* stats;          // [kStatDropped] += dropped keys (atomically: views run together)
   uint64_t* keys;         // cap: the scattered keys
-  uint64_t* tmp;          // cap: merge scratch of segments over 1024 keys
+  uint64_t* tmp;          // cap: the buckets of segments over 1024 keys, and merge scratch
   uint32_t* ids;          // cap: the raster values in sorted order
 };
 
@@ -172,8 +172,9 @@ struct RasterBufs {
   float* T;
   uint32_t* end;
   float4* gC;             // dL/dC, w = valid
-  uint64_t* took;         // per 64-key chunk of a tile and 4x4 pixels: the keys that one of the pixels took
-                          // (training: written by the forward, read by the backward)
+  uint64_t* took;         // per 64-key chunk of a tile and 4x4 pixels: the keys that one of the pixels took, or
+                          // in the first word of each four those that one of the wave's did (training: written
+                          // by the forward, read by the backward)
   const uint32_t* tgt;    // packed RGBA8 targets (all views)
   double* stats;          // kStatDoubles, or null
 };
@@ -247,19 +248,20 @@ bool raster_shape_ok(int tile, int batch);
 // `keys` sorted keys
 size_t raster_took_bytes(int tile, int w, int h, int64_t keys);
 
-// loss: 0 none (view render), 1 Charbonnier fused into the forward pass,
-// 2 forward only, loss computed by a separate kernel
+// loss: 0 none (view render), 1 Charbonnier fused into the forward pass
+// (statistics and dL/dC; no backward can follow), 2 forward only, for a loss
+// computed by a separate kernel: records the taken keys (RasterBufs::took)
 void launch_raster_fwd(hipStream_t st, const RasterShape& sh, const Cam& cam, const Cut& cut, const RasterBufs& b,
                        int loss);
 void launch_loss_l1ssim(hipStream_t st, const Cam& cam, float lambda, const RasterBufs& b,
                         float* scratch);
+// Backward of a forward with loss 2, whose taken keys it walks.
 // boundedColourGrad: every |dL/dC| * 16384 is far below 1e9 (the
 // Charbonnier loss), so the colour terms skip the fixed-point clamp
 void launch_raster_bwd(hipStream_t st, const RasterShape& sh, const Cam& cam, const Cut& cut, const RasterBufs& b,
                        int accumMode, void* accum, bool boundedColourGrad);
 // forward with the Charbonnier loss and backward of a training step in one
-// launch (the same results as launch_raster_fwd with loss 1, then
-// launch_raster_bwd)
+// launch; its image and statistics are those of launch_raster_fwd with loss 1
 void launch_raster_fwd_bwd(hipStream_t st, const RasterShape& sh, const Cam& cam, const Cut& cut, const RasterBufs& b,
                            int accumMode, void* accum, bool boundedColourGrad);
 
@@ -267,9 +269,9 @@ void launch_update(hipStream_t st, int deg, int accumMode, int prec, const Cam& 
                    const UpdateBufs& u);
 
 // Batched views: the projection of view v with its camera from vb->cams[v];
-// one persistent forward and one persistent backward launch over every
-// view's tiles (queue: a counter zeroed before each launch; blocks from
-// raster_views_blocks); one update that chains each view's sums through
+// one persistent launch of forward and backward over every view's tiles
+// (queue: a counter zeroed before it; blocks from raster_views_blocks); one
+// update that chains each view's sums through
 // its camera, adds the views' gradients and takes one Adam step (vb->hp).
 // every view's projection in one launch, into vb->seg[v]'s buffers
 void launch_project_views(hipStream_t st, int deg, int prec, int64_t n, int64_t cap, const ViewBlock* vb, int V,
@@ -321,7 +323,6 @@ struct RefineOp {
   int32_t pad;
 };
 
-// q[i] = (opacity logit, log-scale x, y, z) for i < n
 // Copies the statistics src to out (pinned), clears window's loss sums, src too
 // where clearSrc, and camWords words of camGrad.
 void launch_stats_read(hipStream_t st, double* src, double* window, double* out, bool clearSrc, uint32_t* camGrad,
@@ -334,6 +335,7 @@ void launch_param_rows(hipStream_t st, int64_t cap, int64_t first, int64_t count
 void launch_sh_rows(hipStream_t st, int fmt, int64_t cap, int64_t first, int64_t count, int C, const void* SH,
                     float* out);
 
+// q[i] = (opacity logit, log-scale x, y, z) for i < n
 void launch_refine_gather(hipStream_t st, int64_t n, int64_t cap, const float4* P, float4* q);
 void launch_refine_apply(hipStream_t st, int deg, int prec, int64_t cap, const RefineOp* ops, int64_t count,
                          float4* P, void* M, void* V, void* SH, void* SHM, void* SHV);

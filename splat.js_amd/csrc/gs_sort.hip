@@ -501,14 +501,14 @@ void launch_fill_u32(hipStream_t st, uint32_t* p, int64_t count, uint32_t v) {
 // segment by (depth, id), the reference's order (shaders.js:454), whatever
 // order the scatter left it in.
 //
-// No global atomics: blocks of kSegGroup Gaussians count their keys per tile
-// in an LDS histogram and write it as one row of a [block][tile] table; a
-// column scan turns the table into each block's offset inside every tile's
-// segment (and the tile totals); the scatter then places keys with LDS
-// counters only. A segment of up to 1024 keys sorts in one block: 256-key
-// runs by single waves (bitonic through lane shuffles), then up to two LDS
-// merge levels; longer segments sort 1024-key runs that way and merge them
-// pairwise in global memory.
+// No global atomics: blocks of Gaussians (up to 256, of equal cost) count
+// their keys per tile in an LDS histogram and write it as one row of a
+// [block][tile] table; a column scan turns the table into each block's offset
+// inside every tile's segment (and the tile totals); the scatter then places
+// keys with LDS counters only, dense views in bands of tile rows. A segment
+// of up to 1024 keys sorts in one block: 256-key runs by single waves (bitonic
+// through lane exchanges), then up to two LDS merge levels; longer segments
+// are split into buckets that sort that way.
 
 constexpr int kSegThreads = 1024;     // threads of the count and scatter blocks
 // per-tile LDS arrays (histogram, counters, scan input) are sized to the
