@@ -30,14 +30,15 @@
 #include "gs_math.h"
 
 // tile rows per band for `keys` keys of n Gaussians, scattered by nb blocks
-// into tilesX x tilesY tiles; tilesY: one band
-GS_HD int gs_band_rows(uint64_t keys, int64_t n, int nb, int tilesX, int tilesY) {
+// into numTiles tiles, tilesX to a row; 0: one band (sparse views, most of
+// them, leave before the first division: each costs a block some 20 cycles)
+GS_HD int gs_band_rows(uint64_t keys, int64_t n, int nb, int tilesX, int numTiles) {
   const int lines = (3 << 20) / 128;   // open lines per XCD
-  const int fit = lines / ((nb + 7) / 8) / tilesX, rows = fit < 1 ? 1 : fit < tilesY ? fit : tilesY;
+  if (keys < (uint64_t)12 * (uint64_t)nb * (uint64_t)numTiles) return 0;
+  const int tilesY = numTiles / tilesX, fit = lines / ((nb + 7) / 8) / tilesX, rows = fit < 1 ? 1 : fit;
+  if (rows >= tilesY) return 0;
   const int64_t bands = (tilesY + rows - 1) / rows, walked = n - (1 << 19);
-  if (keys < (uint64_t)12 * (uint64_t)nb * (uint64_t)tilesX * (uint64_t)tilesY) return tilesY;
-  if (walked > 0 && keys < (uint64_t)(3 * bands * walked)) return tilesY;
-  return rows;
+  return walked > 0 && keys < (uint64_t)(3 * bands * walked) ? 0 : rows;
 }
 
 #endif

@@ -609,8 +609,8 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
   int lastKey = 0;                           // fixed: of the group this lane adds for
   const int keyFrom = 4 * 16 * (lane & 3);   // a lane of it, as ds_bpermute counts
   uint32_t lastId = 0;                       // f32: the Gaussian of the last visit
-  const int grp = lane >> 4;
-  uint8_t* const list = sList + (wv * kGroups + grp) * kKeys;
+  uint8_t* const lists = sList + wv * kGroups * kKeys;        // the wave's
+  const uint8_t* const list = lists + (lane >> 4) * kKeys;    // this lane's group's
   float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float Ta = 0.0f;
   uint32_t myEnd = s;
@@ -666,18 +666,19 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
       }
     }
   };
-  // One visit, straight-line for all 64 lanes: the record at LDS offset jo
-  // from the three arrays' starts a0, b0 and c0; `before`: the key lies
-  // before this lane's end. Lanes that do not take the splat (outside the
+  // One visit, straight-line for all 64 lanes: the record at LDS offset
+  // offset() from the three arrays' starts a0, b0 and c0 (behind the reads of
+  // the previous visit's words); before(): the key lies before this lane's end. Lanes that do not take the splat (outside the
   // image, past their `end`, outside the cutoff, alpha below A_MIN, their
   // group past its list) keep their state and contribute zero terms. Some
   // lane took the splat in the forward, so there is nothing to vote on.
   // add(w8): the previous visit's words to its sums; ready(): ahead of this
   // visit's reduction. Returns the record's id.
-  const auto visit = [&](const float4* a0, const float4* b0, const float4* c0, uint32_t jo, bool before,
+  const auto visit = [&](const float4* a0, const float4* b0, const float4* c0, auto&& offset, auto&& before,
                          auto&& add, auto&& ready) __attribute__((always_inline)) {
     AccT w8[8];
     red.read(w8);   // the previous visit's words
+    const uint32_t jo = offset();
     const float4 a = lds_at<float4>(a0, jo);
     const float4 bb = lds_at<float4>(b0, jo);   // C, opa*comp, -0.5 cnorm, id
     const float dx = px - a.x, dy = py - a.y;
@@ -688,7 +689,7 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
     const float G = gs_expf_raster(-e);
     const float araw = bb.y * G;
     const float alpha = fminf(0.99f, araw);
-    const bool contrib = before && e <= cut.eCut && alpha >= cut.aMin;
+    const bool contrib = before() && e <= cut.eCut && alpha >= cut.aMin;
     const float4 c4 = lds_at<float4>(c0, jo);
     // Tb = Ta / (1 - alpha), S / (1 - alpha) through one reciprocal.
     // 1 - alpha lies in [0.0099, 1] (alpha in [0, 0.99]); on [2^-9, 1]
@@ -792,7 +793,7 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
       constexpr uint32_t kNone = 0x01010101u * (uint32_t)kKeys;
       int have[kGroups] = {};
       for (int k = lane; k < kGroups * kKeys / 8; k += 64)
-        reinterpret_cast<uint2*>(sList + wv * kGroups * kKeys)[k] = make_uint2(kNone, kNone);
+        reinterpret_cast<uint2*>(lists)[k] = make_uint2(kNone, kNone);
 #pragma unroll
       for (int c = kKeys / 64 - 1; c >= 0; c--) {
 #pragma unroll
@@ -803,7 +804,7 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
           const int cnt = __builtin_popcountll(m);
           const uint32_t below = __builtin_amdgcn_mbcnt_hi(mHi, __builtin_amdgcn_mbcnt_lo(mLo, 0u));
           if (__builtin_amdgcn_inverse_ballot_w64(m))
-            list[kKeys * (q - grp) + have[q] + cnt - 1 - (int)below] = (uint8_t)(64 * c + lane);
+            lists[kKeys * q + have[q] + cnt - 1 - (int)below] = (uint8_t)(64 * c + lane);
           have[q] += cnt;
         }
       }
@@ -811,9 +812,14 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
       if (steps != 0) {
         int nextKey = (int)list[0];
         for (int step = 0; step < steps; step++) {
-          const int key = nextKey;
-          nextKey = (int)list[step + 1 < kKeys ? step + 1 : 0];
-          visit(sA, sB, sC, (uint32_t)key * 16u, key < pastEnd,
+          int key = 0;
+          visit(sA, sB, sC,
+                [&]() {
+                  key = nextKey;
+                  nextKey = (int)list[step + 1 < kKeys ? step + 1 : 0];
+                  return (uint32_t)key * 16u;
+                },
+                [&]() { return key < pastEnd; },
                 [&](const AccT* w8) { add_group_sums(sSum, lastKey, red.slot, red.total(w8), red.flusher); },
                 // the next key has arrived by now: waited for here, not behind the writes
                 [&]() { asm volatile("" : "+v"(nextKey)); });
@@ -842,7 +848,8 @@ __device__ __forceinline__ void raster_bwd_tile(const Cam& cam, const Cut& cut, 
           const int bit = 63 - __builtin_clzll(m);
           clear_bit(m, bit);
           const uint32_t id =
-              visit(sA + 64 * c, sB + 64 * c, sC + 64 * c, lds_offset((uint32_t)bit * 16u), bit < past,
+              visit(sA + 64 * c, sB + 64 * c, sC + 64 * c, [&]() { return lds_offset((uint32_t)bit * 16u); },
+                    [&]() { return bit < past; },
                     [&](const AccT* w8) {
                       add_wave_sums((float*)accum, lastId, red.slot, red.wave_total(w8), red.flusher && (lane & 3) == 0);
                     },

@@ -1014,8 +1014,8 @@ struct ScatterPrep {
 
 // the scatter's bands of tile rows (gs_bands.h)
 __device__ __forceinline__ SegBands seg_bands(const SegJob& j) {
-  const int tilesY = j.numTiles / j.tilesX;
-  return {tilesY, gs_band_rows(*j.totalKeys, j.n, j.nb, j.tilesX, tilesY)};
+  const int rows = gs_band_rows(*j.totalKeys, j.n, j.nb, j.tilesX, j.numTiles);
+  return rows ? SegBands{j.numTiles / j.tilesX, rows} : SegBands{1, 1};
 }
 
 // Every (Gaussian, kept tile) key into its tile's segment: each tile's LDS
